@@ -23,7 +23,6 @@ double fsm_batch(st_ctx *ctx, const float *dsrc, const float *hsrc, int nshot, c
 void fsm_pad(st_ctx *ctx, float *S);
 void fsm_picks(st_ctx *ctx, int nshot, const float *drcv, int nrcv, float *dpicks);
 void fsm_crop_volumes(st_ctx *ctx, float *dout, int nshot);
-int fsm_lanes(int nshot);
 void launch_extract(st_ctx *ctx, float *dout, int nshot, int B);
 void launch_picks_blk(hipStream_t st, const float *T, long long vol, int nshot, const float *rcv,
                       int nr, float *out, int nx, int ny, int nz, float dx, float dy, float dz,
@@ -62,8 +61,8 @@ void tomo_trace_blk(st_ctx *ctx, const float *T, long long vol, int B, int nbx, 
                     const float *dsrc, int nshot, const float *drcv, int nr, bool with_illum);
 void tomo_trace_zxy(st_ctx *ctx, const float *dT, const float *dsrc, const float *drcv, int nr,
                     bool with_illum);
-void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, int cell_stride,
-                    const float *dsrc, int nshot, const float *drcv, int nr, bool with_illum);
+void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, const float *dsrc,
+                    int nshot, const float *drcv, int nr, bool with_illum);
 void tomo_get_illum(st_ctx *ctx, float *out);
 void tomo_csr(st_ctx *ctx, long long *rows, long long *nnz, const long long **rp, const int **c,
               const float **v);
@@ -350,8 +349,8 @@ static int fsm_setup(st_ctx *ctx, int nshot, int batch, bool with_T_out) {
     ST_HIP(hipMemGetInfo(&free_b, &total_b));
     const size_t per_shot = sizeof(float) * nB + (with_T_out ? sizeof(float) * npts : 0);
     const size_t have = free_b + ctx->T.bytes + ctx->scratch.bytes;
-    while (b > 1 && per_shot * (size_t)fsm_lanes(b) > have / 2) b /= 2;
-    ctx->T.reserve(sizeof(float) * nB * fsm_lanes(b));
+    while (b > 1 && per_shot * (size_t)b > have / 2) b /= 2;
+    ctx->T.reserve(sizeof(float) * nB * b);
     if (with_T_out) ctx->scratch.reserve(sizeof(float) * npts * b);
     return b;
 }
@@ -897,7 +896,8 @@ static void forward_impl(st_ctx *ctx, const float *src_xyz, int nshot, const flo
             }
         }
     } else if (type == 2) {
-        // Accurate_FSM: the padded, shot-fastest volumes are traced in place
+        // Accurate_FSM: the padded volumes are traced in place
+        const long long nB = (long long)(ctx->nx + 2) * (ctx->ny + 2) * (ctx->nz + 2);
         const int b = fsm_setup(ctx, nshot, o.batch, T_out != nullptr);
         for (int b0 = 0; b0 < nshot; b0 += b) {
             const int nb = std::min(b, nshot - b0);
@@ -905,7 +905,7 @@ static void forward_impl(st_ctx *ctx, const float *src_xyz, int nshot, const flo
             const double t = fsm_batch(ctx, dsrc, src_xyz + 3LL * b0, nb, ctx->fsm_S.as<float>());
             if (stats) { stats->solve_ms += t; stats->batches += 1; }
             fsm_picks(ctx, nb, drcv, nrcv, ctx->picks.as<float>() + (long long)b0 * nrcv);
-            tomo_trace_pad(ctx, ctx->T.as<float>(), 1, fsm_lanes(nb), dsrc, nb, drcv, nrcv, true);
+            tomo_trace_pad(ctx, ctx->T.as<float>(), nB, dsrc, nb, drcv, nrcv, true);
             if (T_out) {
                 fsm_crop_volumes(ctx, ctx->scratch.as<float>(), nb);
                 to_host(b0, nb);
@@ -922,7 +922,7 @@ static void forward_impl(st_ctx *ctx, const float *src_xyz, int nshot, const flo
             if (stats) { stats->solve_ms += t; stats->batches += 1; }
             podvin_picks(ctx, ctx->pod_T.as<float>(), nb, drcv, nrcv,
                          ctx->picks.as<float>() + (long long)b0 * nrcv);
-            tomo_trace_pad(ctx, ctx->pod_T.as<float>(), nB, 1, dsrc, nb, drcv, nrcv, true);
+            tomo_trace_pad(ctx, ctx->pod_T.as<float>(), nB, dsrc, nb, drcv, nrcv, true);
             if (T_out) {
                 podvin_crop_volumes(ctx, ctx->pod_T.as<float>(), ctx->scratch.as<float>(), nb);
                 to_host(b0, nb);

@@ -240,12 +240,6 @@ constexpr float kKeyInf = __builtin_inff();  // "no key" for the arrival orderin
 // s_barrier (which would couple waves with different trip counts).
 constexpr int kWaves = 2;
 
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Segment lengths of this round's list: lane k < kSeg gets the inclusive
 // prefix over segments 0..k in incl, every lane the total in count.
 __device__ __forceinline__ void round_counts(const FimArgs &A, int lane, unsigned &incl,

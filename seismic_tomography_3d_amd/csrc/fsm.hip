@@ -9,32 +9,46 @@
 // sweep's box by p = a + b + c, their distances from the box's start corner
 // along z, x, y.  Every upwind neighbour has a smaller p, and the loop nest
 // (k outer, j, i inner) also visits every cell after all cells of smaller p
-// that it reads.  So updating the planes p = 0, 1, 2, ... one after another,
-// all cells of a plane at once (they read nothing from each other), gives
-// each update the same inputs, and with the same arithmetic the same
-// result.  One kernel launch per plane (kernel boundaries order the planes);
-// a launch covers that plane for every shot of the batch.
+// that it reads.  So any schedule that updates a cell after its upwind
+// neighbours gives each update the same inputs, and with the same arithmetic
+// the same result.
 //
-// Layout: travel times are stored shot-fastest, T[cell * NS + shot] (NS =
-// the batch rounded up to 64), so a wave updates one cell for 64 shots: its
-// T loads are contiguous 256-byte rows and every slowness load and index
-// is wave-uniform.  That needs one cell per plane for all shots, while the
-// eight source-bounded sweeps of init_sweep start at each shot's own source:
-// planes are therefore numbered from the corner of the union of the shots'
-// boxes, and a lane skips cells outside its shot's box.  Within one shot's
-// box the absolute plane number is its own p plus a constant, so the order
-// argument above holds per shot.
+// Schedule: a sweep's box is cut into blocks of 8 x 8 columns (x, y) by a
+// chunk of z, and the blocks with equal A + B + C (block distances from the
+// start corner) are one launch; a block's upwind neighbours lie in blocks of
+// earlier launches or in itself.  One wave updates one block of one shot: lane
+// (x, y) walks its column and is x + y steps behind lane (0, 0), so that at
+// each step the wave updates a diagonal plane of the block and every lane's
+// upwind neighbours were updated in earlier steps.  The block and its upwind
+// halo sit in LDS while the wave works on it (travel times and slowness read
+// once per block, in rows along z), the values along z stay in registers.
+// Each shot's source-bounded sweeps cover that shot's own boxes only.
 //
-// Compiled with -ffp-contract=off and HIP's correctly rounded division and
-// square root; min/max follow std::min/std::max operand order.  The seeds'
-// powf(x, 2.0f) are computed as x*x, the form the reference's compiler
-// emits for them (exact squares; the oracle's CPU build agrees bit for bit).
+// What bounds it: a step of the walk is about 100 (operators ruled out) to 240
+// dependent vector instructions, 400 to 1,000 cycles of one wave, so a lone
+// shot pays (blocks along the longest diagonal) x (zc + 15) such steps per
+// sweep, and a batch the vector issue of the lanes a block's skew leaves busy
+// (zc of zc + 15 steps).  Measured: one shot of 121 x 97 x 61 cells 21.1 ->
+// 6.5 ms, 64 shots of 201 x 201 x 101 77.5 -> 39.2 ms, against a launch per
+// plane of cells with the shots of a batch in the lanes.  Blocks of 14 cells
+// of z: 8 / 14 / 22 / 30 take 45 / 39 / 40 / 43 ms for the 64 shots (the tiles'
+// LDS against the idle lanes) and 7.2 / 7.4 / 7.9 / 7.8 for the lone one.
+//
+// Layout: one padded volume per shot, z fastest.
+//
+// Compiled with -ffp-contract=off and HIP's correctly rounded square root;
+// divisions by the spacing constants are correctly rounded without a divide
+// (div_rn); min/max follow std::min/std::max operand order where a NaN could
+// reach them.  The seeds' powf(x, 2.0f) are computed as x*x, the form the
+// reference's compiler emits for them (exact squares; the oracle's CPU build
+// agrees bit for bit).
 #include "st_common.hpp"
 
 namespace st {
 
-void launch_picks_pad(hipStream_t st, const float *T, int NS, int nshot, const float *rcv, int nr,
-                      float *out, int nx, int ny, int nz, float dx, float dy, float dz);
+void launch_picks_padvol(hipStream_t st, const float *T, long long vol, int nshot,
+                         const float *rcv, int nr, float *out, int nx, int ny, int nz, float dx,
+                         float dy, float dz);
 
 __device__ __forceinline__ float smin(float a, float b) { return (b < a) ? b : a; }
 __device__ __forceinline__ float smax(float a, float b) { return (a < b) ? b : a; }
@@ -46,6 +60,10 @@ struct FsmGeo {
     long long nB;           // nxx * nyy * nzz
     float dx, dy, dz;
     float dz2i, dx2i, dy2i, dz2dx2, dz2dy2, dx2dy2, dsum;
+    float zx, zy, xy;       // dz2i + dx2i, dz2i + dy2i, dx2i + dy2i
+    float rzx, rzy, rxy, rdsum;   // correctly rounded reciprocals of those and dsum
+    float dmin;             // 0.99 of the least spacing
+    float wv, we, wn, wev, wen, wnv;   // weights of the upwind times in the mean of the 3D arms
 };
 
 // One sweep: directions (1 forward, -1 backward) for z (i), x (j), y (k),
@@ -73,79 +91,67 @@ __host__ __device__ inline void sweep_axis(int t, int init, int n, int sid, int 
     }
 }
 
-// The update of one cell, accurate_FSM.cpp:159-265 (inner_sweep).
-__device__ __forceinline__ void fsm_update(float *__restrict__ T, int NS,
-                                           const float *__restrict__ S, const FsmGeo &g, int i,
-                                           int j, int k, int sgntz, int sgntx, int sgnty) {
-    const int sgnvz = (sgntz + 1) >> 1, sgnvx = (sgntx + 1) >> 1, sgnvy = (sgnty + 1) >> 1;
-    const int nzz = g.nzz, nxx = g.nxx, nyy = g.nyy;
-    const long long NZ = nzz, NXZ = (long long)nxx * nzz;
+// Upwind travel times of a cell (v along z, e along x, n along y and their
+// combinations) and the slownesses of its operators: the least of the four
+// voxels around each upwind edge (sv, se, sn), of the two voxels on each
+// upwind face (sve, svn, sen) and the upwind voxel (s).
+struct FsmIn {
+    float tv, te, tn, tev, ten, tnv, tnve;
+    float sv, se, sn, sve, svn, sen, s;
+};
+
+// Least of floats that are never negative nor NaN: their bit patterns order as
+// integers, and an integer minimum needs no quieting of its operands.
+__device__ __forceinline__ float pmin(float a, float b) {
+    return __int_as_float(min(__float_as_int(a), __float_as_int(b)));
+}
+__device__ __forceinline__ float pmax(float a, float b) {
+    return __int_as_float(max(__float_as_int(a), __float_as_int(b)));
+}
+
+// The arms of the 3D operator.  Products with 0.5 are exact, so the fused
+// forms round as the separate ones do.
+__device__ __forceinline__ void fsm_arms(const FsmIn &c, float &ta, float &tb, float &tc) {
+    auto half = [](float a, float b) { return __builtin_fmaf(0.5f, a, b); };
+    ta = half(c.tev, half(-c.tv, half(c.ten, half(-c.tn, c.te)))) - c.tnv + c.tnve;
+    tb = half(c.tev, half(-c.te, half(c.tnv, half(-c.tn, c.tv)))) - c.ten + c.tnve;
+    tc = half(c.tnv, half(-c.tv, half(c.ten, half(-c.te, c.tn)))) - c.tev + c.tnve;
+}
+
+// The update of one cell, accurate_FSM.cpp:159-265 (inner_sweep), as written
+// there.
+__device__ float fsm_update_any(float T, const FsmIn &c, const FsmGeo &g) {
     const float dx = g.dx, dy = g.dy, dz = g.dz;
-    const int i1 = i - sgnvz, j1 = j - sgnvx, k1 = k - sgnvy;
-    const int jm = max(j - 1, 1), jc = min(j, nxx - 1);
-    const int km = max(k - 1, 1), kc = min(k, nyy - 1);
-    const int im = max(i - 1, 1), ic = min(i, nzz - 1);
-
-    // T points at this lane's shot; cells are NS floats apart
-    auto tat = [&](long long c) { return T[c * NS]; };
-    const float tv = tat((i - sgntz) + j * NZ + k * NXZ);
-    const float te = tat(i + (j - sgntx) * NZ + k * NXZ);
-    const float tn = tat(i + j * NZ + (k - sgnty) * NXZ);
-    const float tev = tat((i - sgntz) + (j - sgntx) * NZ + k * NXZ);
-    const float ten = tat(i + (j - sgntx) * NZ + (k - sgnty) * NXZ);
-    const float tnv = tat((i - sgntz) + j * NZ + (k - sgnty) * NXZ);
-    const float tnve = tat((i - sgntz) + (j - sgntx) * NZ + (k - sgnty) * NXZ);
-    const long long ijk = (i + j * NZ + k * NXZ) * NS;
-
-    // 1D operators: upwind time plus spacing times the least of the four
-    // slownesses around the edge
-    const float t1D1 = tv + dz * smin(S[i1 + jm * NZ + km * NXZ],
-                                 smin(S[i1 + jm * NZ + kc * NXZ],
-                                 smin(S[i1 + jc * NZ + km * NXZ], S[i1 + jc * NZ + kc * NXZ])));
-    const float t1D2 = te + dx * smin(S[im + j1 * NZ + km * NXZ],
-                                 smin(S[ic + j1 * NZ + km * NXZ],
-                                 smin(S[im + j1 * NZ + kc * NXZ], S[ic + j1 * NZ + kc * NXZ])));
-    const float t1D3 = tn + dy * smin(S[im + jm * NZ + k1 * NXZ],
-                                 smin(S[im + jc * NZ + k1 * NXZ],
-                                 smin(S[ic + jm * NZ + k1 * NXZ], S[ic + jc * NZ + k1 * NXZ])));
-    const float t1D = smin(t1D1, smin(t1D2, t1D3));
-
+    const float tv = c.tv, te = c.te, tn = c.tn;
+    // 1D operators: upwind time plus spacing times the least slowness
+    const float t1D = smin(tv + dz * c.sv, smin(te + dx * c.se, tn + dy * c.sn));
     // 2D four-point operators in the xz, yz and xy planes
     float t2D1 = 1e6f, t2D2 = 1e6f, t2D3 = 1e6f;
-    float Sref = smin(S[i1 + j1 * NZ + km * NXZ], S[i1 + j1 * NZ + kc * NXZ]);
-    if ((tv < te + dx * Sref) && (te < tv + dz * Sref)) {
-        const float ta = tev + te - tv;
-        const float tb = tev - te + tv;
+    if ((tv < te + dx * c.sve) && (te < tv + dz * c.sve)) {
+        const float ta = c.tev + te - tv;
+        const float tb = c.tev - te + tv;
         t2D1 = ((tb * g.dz2i + ta * g.dx2i) +
-                sqrtf(4.0f * Sref * Sref * (g.dz2i + g.dx2i) -
-                      g.dz2i * g.dx2i * (ta - tb) * (ta - tb))) / (g.dz2i + g.dx2i);
+                sqrtf(4.0f * c.sve * c.sve * g.zx - g.dz2dx2 * (ta - tb) * (ta - tb))) / g.zx;
     }
-    Sref = smin(S[i1 + jm * NZ + k1 * NXZ], S[i1 + jc * NZ + k1 * NXZ]);
-    if ((tv < tn + dy * Sref) && (tn < tv + dz * Sref)) {
-        const float ta = tv - tn + tnv;
-        const float tb = tn - tv + tnv;
+    if ((tv < tn + dy * c.svn) && (tn < tv + dz * c.svn)) {
+        const float ta = tv - tn + c.tnv;
+        const float tb = tn - tv + c.tnv;
         t2D2 = ((ta * g.dz2i + tb * g.dy2i) +
-                sqrtf(4.0f * Sref * Sref * (g.dz2i + g.dy2i) -
-                      g.dz2i * g.dy2i * (ta - tb) * (ta - tb))) / (g.dz2i + g.dy2i);
+                sqrtf(4.0f * c.svn * c.svn * g.zy - g.dz2dy2 * (ta - tb) * (ta - tb))) / g.zy;
     }
-    Sref = smin(S[im + j1 * NZ + k1 * NXZ], S[ic + j1 * NZ + k1 * NXZ]);
-    if ((te < tn + dy * Sref) && (tn < te + dx * Sref)) {
-        const float ta = te - tn + ten;
-        const float tb = tn - te + ten;
+    if ((te < tn + dy * c.sen) && (tn < te + dx * c.sen)) {
+        const float ta = te - tn + c.ten;
+        const float tb = tn - te + c.ten;
         t2D3 = ((ta * g.dx2i + tb * g.dy2i) +
-                sqrtf(4.0f * Sref * Sref * (g.dx2i + g.dy2i) -
-                      g.dx2i * g.dy2i * (ta - tb) * (ta - tb))) / (g.dx2i + g.dy2i);
+                sqrtf(4.0f * c.sen * c.sen * g.xy - g.dx2dy2 * (ta - tb) * (ta - tb))) / g.xy;
     }
     const float t2D = smin(t2D1, smin(t2D2, t2D3));
-
     // 3D operator on the upwind octant
     float t3D = 1e6f;
-    Sref = S[i1 + j1 * NZ + k1 * NXZ];
-    const float ta = te - 0.5f * tn + 0.5f * ten - 0.5f * tv + 0.5f * tev - tnv + tnve;
-    const float tb = tv - 0.5f * tn + 0.5f * tnv - 0.5f * te + 0.5f * tev - ten + tnve;
-    const float tc = tn - 0.5f * te + 0.5f * ten - 0.5f * tv + 0.5f * tnv - tev + tnve;
     if (smin(t1D, t2D) > smax(tv, smax(te, tn))) {
-        const float t2 = 9.0f * Sref * Sref * g.dsum;
+        float ta, tb, tc;
+        fsm_arms(c, ta, tb, tc);
+        const float t2 = 9.0f * c.s * c.s * g.dsum;
         const float t3 = g.dz2dx2 * (ta - tb) * (ta - tb) + g.dz2dy2 * (tb - tc) * (tb - tc) +
                          g.dx2dy2 * (ta - tc) * (ta - tc);
         if (t2 >= t3) {
@@ -153,7 +159,85 @@ __device__ __forceinline__ void fsm_update(float *__restrict__ T, int NS,
             t3D = (t1 + sqrtf(t2 - t3)) / g.dsum;
         }
     }
-    T[ijk] = smin(T[ijk], smin(t1D, smin(t2D, t3D)));
+    return smin(T, smin(t1D, smin(t2D, t3D)));
+}
+
+// The same update, bit for bit, in the ranges fsm_fast checks: square roots
+// and quotients by the spacing constants in their short correctly rounded
+// forms, and operators that cannot change the result left out.  With lim the
+// least of the cell's time and the 1D operators:
+// * t3D is at least the weighted mean of its arms (its root is not negative
+//   and rounding is monotone), a linear form of the seven upwind times; above
+//   lim by more than rounding (2^-17 of the times) it is ruled out;
+// * a 2D operator is at least its diagonal time plus the slowness times the
+//   lesser spacing (its root term is concave in the difference of the two
+//   axis times, with the spacings' values at the ends of the admitted range);
+//   with 1 % of that term and 2^-16 of lim for rounding, at or above lim it
+//   is ruled out -- unless the 3D operator is in play, whose condition reads
+//   the 2D times.
+// In most of the sixteen sweeps a cell's front does not come from the sweep's
+// octant, and the operators fall away for whole waves.
+//
+// Branches are wave-uniform (any lane needs the operator), the lanes that do
+// not are masked by selects: a walk's steps depend on each other, and masked
+// branches cost more latency there than the instructions they skip.
+__device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool on,
+                                                 const FsmGeo &g) {
+    const float dx = g.dx, dy = g.dy, dz = g.dz;
+    const float tv = c.tv, te = c.te, tn = c.tn;
+    const float t1D = pmin(tv + dz * c.sv, pmin(te + dx * c.se, tn + dy * c.sn));
+    const float latest = pmax(tv, pmax(te, tn));
+    const float lim = pmin(T, t1D);
+    float l3 = __builtin_fmaf(g.wv, tv, c.tnve);
+    l3 = __builtin_fmaf(g.we, te, l3);
+    l3 = __builtin_fmaf(g.wn, tn, l3);
+    l3 = __builtin_fmaf(g.wev, c.tev, l3);
+    l3 = __builtin_fmaf(g.wen, c.ten, l3);
+    l3 = __builtin_fmaf(g.wnv, c.tnv, l3);
+    const float big = pmax(pmax(latest, c.tnve), pmax(c.tev, pmax(c.ten, c.tnv)));
+    const bool try3 = on & (t1D > latest) & (l3 < __builtin_fmaf(big + lim, 7.6293945e-6f, lim));
+    const float far2 = lim * 1.0000153f;
+    const bool pxz = try3 | (on & (__builtin_fmaf(c.sve, g.dmin, c.tev) < far2));
+    const bool pyz = try3 | (on & (__builtin_fmaf(c.svn, g.dmin, c.tnv) < far2));
+    const bool pxy = try3 | (on & (__builtin_fmaf(c.sen, g.dmin, c.ten) < far2));
+    float t2D = 1e6f;
+    if (__any(pxz)) {
+        const bool ok = pxz & (tv < te + dx * c.sve) & (te < tv + dz * c.sve);
+        const float ta = c.tev + te - tv;
+        const float tb = c.tev - te + tv;
+        const float q = 4.0f * c.sve * c.sve * g.zx - g.dz2dx2 * (ta - tb) * (ta - tb);
+        const float t = div_rn((tb * g.dz2i + ta * g.dx2i) + sqrt_rn(q), g.zx, g.rzx);
+        t2D = ok ? t : t2D;
+    }
+    if (__any(pyz)) {
+        const bool ok = pyz & (tv < tn + dy * c.svn) & (tn < tv + dz * c.svn);
+        const float ta = tv - tn + c.tnv;
+        const float tb = tn - tv + c.tnv;
+        const float q = 4.0f * c.svn * c.svn * g.zy - g.dz2dy2 * (ta - tb) * (ta - tb);
+        const float t = div_rn((ta * g.dz2i + tb * g.dy2i) + sqrt_rn(q), g.zy, g.rzy);
+        t2D = ok & (t < t2D) ? t : t2D;
+    }
+    if (__any(pxy)) {
+        const bool ok = pxy & (te < tn + dy * c.sen) & (tn < te + dx * c.sen);
+        const float ta = te - tn + c.ten;
+        const float tb = tn - te + c.ten;
+        const float q = 4.0f * c.sen * c.sen * g.xy - g.dx2dy2 * (ta - tb) * (ta - tb);
+        const float t = div_rn((ta * g.dx2i + tb * g.dy2i) + sqrt_rn(q), g.xy, g.rxy);
+        t2D = ok & (t < t2D) ? t : t2D;
+    }
+    float res = smin(lim, t2D);
+    const bool use3 = try3 & (smin(t1D, t2D) > latest);
+    if (__any(use3)) {
+        float ta, tb, tc;
+        fsm_arms(c, ta, tb, tc);
+        const float t2 = 9.0f * c.s * c.s * g.dsum;
+        const float t3 = g.dz2dx2 * (ta - tb) * (ta - tb) + g.dz2dy2 * (tb - tc) * (tb - tc) +
+                         g.dx2dy2 * (ta - tc) * (ta - tc);
+        const float t1 = tb * g.dz2i + ta * g.dx2i + tc * g.dy2i;
+        const float t = div_rn(t1 + sqrt_rn(t2 - t3), g.dsum, g.rdsum);
+        res = use3 & (t2 >= t3) & (t < res) ? t : res;
+    }
+    return res;
 }
 
 // Slowness padded by one cell, edge replicated: expand_model
@@ -209,7 +293,7 @@ __constant__ signed char kSeed[27][6] = {
 
 // One thread per shot, the entries in table order (entries that name the
 // same node are written in the reference's order: the last wins).
-__global__ void fsm_seed(float *__restrict__ T, int NS, const float *__restrict__ S,
+__global__ void fsm_seed(float *__restrict__ T, const float *__restrict__ S,
                          const float *__restrict__ src, const int *__restrict__ sid, int nshot,
                          FsmGeo g) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
@@ -219,7 +303,7 @@ __global__ void fsm_seed(float *__restrict__ T, int NS, const float *__restrict_
     const int sidz = sid[3 * s], sidx = sid[3 * s + 1], sidy = sid[3 * s + 2];
     const long long NZ = g.nzz, NXZ = (long long)g.nxx * g.nzz;
     const long long sId = sidz + sidx * NZ + sidy * NXZ;
-    float *Ts = T + s;
+    float *Ts = T + s * g.nB;
     const float S0 = S[sId];
     for (int e = 0; e < 27; e++) {
         const int iz = kSeed[e][0], ix = kSeed[e][1], iy = kSeed[e][2];
@@ -227,44 +311,169 @@ __global__ void fsm_seed(float *__restrict__ T, int NS, const float *__restrict_
         const float ex = ((sidx - nb) + ox) * g.dx - sx;
         const float ey = ((sidy - nb) + oy) * g.dy - sy;
         const float ez = ((sidz - nb) + oz) * g.dz - sz;
-        Ts[(sId + iz + ix * NZ + iy * NXZ) * NS] = S0 * sqrtf(ex * ex + ey * ey + ez * ez);
+        Ts[sId + iz + ix * NZ + iy * NXZ] = S0 * sqrtf(ex * ex + ey * ey + ez * ez);
     }
 }
 
-// One plane p of one sweep for all shots.  The union box of the sweep
-// starts at (zs, xs, ys) and runs along the sweep directions; cells of the
-// plane are enumerated by (a, c) -- distances along z and y -- over the
-// rectangle [a0, a0 + na) x [c0, c0 + nc), with b = p - a - c along x.
-// Thread q: cell q / NS of the rectangle, shot q % NS (waves never straddle
-// cells: NS and the block size are multiples of 64).
-__global__ __launch_bounds__(256) void fsm_plane(float *__restrict__ T, int NS, int nshot,
-                                                 const float *__restrict__ S,
-                                                 const int *__restrict__ sid, FsmGeo g,
-                                                 FsmSweep w, int zs, int xs, int ys, int xl, int p,
-                                                 int a0, int na, int c0, int nc) {
-    const long long q = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const int cell = __builtin_amdgcn_readfirstlane((int)(q / NS));
-    if (cell >= na * nc) return;
-    const int a = a0 + cell % na, c = c0 + cell / na;
-    const int b = p - a - c;
-    if (b < 0 || b >= xl) return;
-    const int s = (int)(q - (long long)cell * NS);
-    if (s >= nshot) return;
-    const int i = zs + w.tz * a, j = xs + w.tx * b, k = ys + w.ty * c;
-    // this shot's own box along each axis
-    int st, ln;
-    sweep_axis(w.tz, w.init, g.nzz, sid[3 * s], st, ln);
-    if (w.tz * (i - st) < 0 || w.tz * (i - st) >= ln) return;
-    sweep_axis(w.tx, w.init, g.nxx, sid[3 * s + 1], st, ln);
-    if (w.tx * (j - st) < 0 || w.tx * (j - st) >= ln) return;
-    sweep_axis(w.ty, w.init, g.nyy, sid[3 * s + 2], st, ln);
-    if (w.ty * (k - st) < 0 || w.ty * (k - st) >= ln) return;
-    fsm_update(T + s, NS, S, g, i, j, k, w.tz, w.tx, w.ty);
+// One diagonal D of one sweep's blocks, for all shots.  Blocks are (A, B, C)
+// = distances from the start corner of the shot's box in units of zc cells
+// along z and eight along x and y; workgroup q holds shot q % nshot of block
+// (a0 + r % na, D - A - C, c0 + r / na), r = q / nshot.  A shot whose box has
+// no such block leaves at once.
+//
+// The LDS tiles hold planes 0 (the upwind halo) .. 8 along x and y and 0 ..
+// zc along z, in sweep order.  P even and Q = 9 mod 16 put the 64 lanes of a
+// step, whose z differ by x + y, on 64 different banks.  Slowness is stored
+// as the voxel on the downwind side of each cell, so a cell's eight voxels
+// are the tile's entries at offsets 0 and -1 per axis: padded voxel i for a
+// forward sweep and i - 1 for a backward one.  The reference's index clamps
+// (max(i - 1, 1), min(i, n - 1)) only choose between a padding voxel and the
+// edge voxel it copies, so clamping at 0 gives the same value.
+constexpr int kFsmZ = 14;   // most z cells of a block
+template <int LZ> struct FsmTile {
+    static constexpr int P = (LZ + 2) & ~1;
+    static constexpr int Q = ((9 * P - 9 + 15) / 16) * 16 + 9;
+    static constexpr int N = 9 * Q;
+};
+
+template <int LZ, bool FAST>
+__global__ __launch_bounds__(64) void fsm_block(float *__restrict__ T,
+                                                const float *__restrict__ S,
+                                                const int *__restrict__ sid, int nshot, FsmGeo g,
+                                                FsmSweep w, int zc, int D, int a0, int na, int c0) {
+    using Tile = FsmTile<LZ>;
+    constexpr int P = Tile::P, Q = Tile::Q;
+    __shared__ float tt[Tile::N + 1];
+    __shared__ float ts[Tile::N];
+    const int shot = blockIdx.x % nshot, r = blockIdx.x / nshot;
+    const int A = a0 + r % na, C = c0 + r / na, B = D - A - C;
+    int zs, zl, xs, xl, ys, yl;
+    sweep_axis(w.tz, w.init, g.nzz, sid[3 * shot], zs, zl);
+    sweep_axis(w.tx, w.init, g.nxx, sid[3 * shot + 1], xs, xl);
+    sweep_axis(w.ty, w.init, g.nyy, sid[3 * shot + 2], ys, yl);
+    if (B < 0 || 8 * B >= xl || 8 * C >= yl || zc * A >= zl) return;
+    float *Ts = T + shot * g.nB;
+    const int lane = threadIdx.x;
+    const int len = min(zc, zl - zc * A);      // z cells of this block
+    const int nb = min(8, xl - 8 * B), nc = min(8, yl - 8 * C);
+    const int z1 = zs + w.tz * (zc * A), x1 = xs + w.tx * (8 * B), y1 = ys + w.ty * (8 * C);
+    const int bz = w.tz < 0, bx = w.tx < 0, by = w.ty < 0;
+
+    // stage: RPW rows along z per load, a plane of y at a time; indices are
+    // clamped into the volume, entries past the box are not used
+    constexpr int RZ = LZ < 16 ? 16 : (LZ < 32 ? 32 : 64), RPW = 64 / RZ;
+    constexpr int NB = (9 + RPW - 1) / RPW;   // loads per plane
+    const int rz = lane & (RZ - 1), row0 = lane / RZ;
+    {
+        const int i = min(max(z1 + w.tz * (rz - 1), 0), g.nzz - 1);
+        const int iv = max(i - bz, 0);
+        int ot[NB], os[NB];
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int j = min(max(x1 + w.tx * (row0 + u * RPW - 1), 0), g.nxx - 1);
+            ot[u] = i + g.nzz * j;
+            os[u] = iv + g.nzz * max(j - bx, 0);
+        }
+        float *t0 = tt + row0 * P + rz, *s0 = ts + row0 * P + rz;
+        float vt[9 * NB], vs[9 * NB];
+#pragma unroll
+        for (int c = 0; c < 9; c++) {
+            const int k = min(max(y1 + w.ty * (c - 1), 0), g.nyy - 1);
+            const float *Tk = Ts + (long long)k * g.nxx * g.nzz;
+            const float *Sk = S + (long long)max(k - by, 0) * g.nxx * g.nzz;
+#pragma unroll
+            for (int u = 0; u < NB; u++) {
+                vt[c * NB + u] = Tk[ot[u]];
+                vs[c * NB + u] = Sk[os[u]];
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        if (rz <= LZ) {
+#pragma unroll
+            for (int c = 0; c < 9; c++)
+#pragma unroll
+                for (int u = 0; u < NB; u++)
+                    if (u * RPW + RPW <= 9 || row0 < 9 - u * RPW) {
+                        t0[c * Q + u * RPW * P] = vt[c * NB + u];
+                        s0[c * Q + u * RPW * P] = vs[c * NB + u];
+                    }
+        }
+    }
+    wave_sync();
+
+    // the walk: lane (x, y) is at z cell a = s - x - y; a = -1 reads the
+    // halo plane into the registers that carry the values along z
+    const int x = lane & 7, y = lane >> 3;
+    int at = (y + 1) * Q + (x + 1) * P - x - y;   // tile index of a, at s = -1
+    // a = at - lo, in [0, len) for the cells of the block
+    const int lo = x < nb && y < nc ? (y + 1) * Q + (x + 1) * P + 1 : 1 << 24;
+    float tv = 0, tev = 0, tnv = 0, tnve = 0;
+    float suu = 0, sxu = 0, syu = 0, s4 = 0;      // upwind voxels: (x, y) up, x up, y up, all four
+    // own time and voxels of the step, read one step ahead (no other lane
+    // writes them)
+    float own = tt[at], vdd = ts[at], vud = ts[at - P], vdu = ts[at - Q], vuu = ts[at - P - Q];
+#pragma unroll 2
+    for (int s = -1; s < len + 14; s++, at++) {
+        FsmIn c;
+        c.te = tt[at - P];
+        c.tn = tt[at - Q];
+        c.ten = tt[at - P - Q];
+        const float own1 = tt[at + 1], vdd1 = ts[at + 1], vud1 = ts[at + 1 - P],
+                    vdu1 = ts[at + 1 - Q], vuu1 = ts[at + 1 - P - Q];
+        c.tv = tv;
+        c.tev = tev;
+        c.tnv = tnv;
+        c.tnve = tnve;
+        const float nxu = pmin(vuu, vud), nyu = pmin(vuu, vdu);
+        c.sv = s4;
+        c.se = pmin(sxu, nxu);
+        c.sn = pmin(syu, nyu);
+        c.sve = sxu;
+        c.svn = syu;
+        c.sen = pmin(suu, vuu);
+        c.s = suu;
+        const bool on = (unsigned)(at - lo) < (unsigned)len;
+        float res = FAST ? fsm_update_fast(own, c, on, g) : fsm_update_any(own, c, g);
+        res = on ? res : own;
+        tt[on ? at : Tile::N] = res;   // the last word takes what is not a cell
+        tv = res;
+        tev = c.te;
+        tnv = c.tn;
+        tnve = c.ten;
+        suu = vuu;
+        sxu = nxu;
+        syu = nyu;
+        s4 = pmin(nxu, pmin(vdu, vdd));
+        own = own1;
+        vdd = vdd1;
+        vud = vud1;
+        vdu = vdu1;
+        vuu = vuu1;
+        wave_sync();
+    }
+
+    // the block back to memory
+    if (rz >= 1 && rz <= len) {
+        const int i = z1 + w.tz * (rz - 1);
+        constexpr int NS = 8 / RPW;
+        int o[NS];
+#pragma unroll
+        for (int u = 0; u < NS; u++) o[u] = i + g.nzz * (x1 + w.tx * (row0 + u * RPW));
+        const float *t0 = tt + Q + (row0 + 1) * P + rz;
+#pragma unroll
+        for (int c = 0; c < 8; c++) {
+            if (c >= nc) break;
+            float *Tk = Ts + (long long)(y1 + w.ty * c) * g.nxx * g.nzz;
+#pragma unroll
+            for (int u = 0; u < NS; u++)
+                if (row0 + u * RPW < nb) Tk[o[u]] = t0[c * Q + u * RPW * P];
+        }
+    }
 }
 
 // reduce_model (accurate_FSM.cpp:62-72): padded -> model extent, z fastest
-__global__ void fsm_crop(const float *__restrict__ T, int NS, float *__restrict__ out, int nx,
-                         int ny, int nz, int nshot) {
+__global__ void fsm_crop(const float *__restrict__ T, float *__restrict__ out, int nx, int ny,
+                         int nz, long long nB, int nshot) {
     const long long npts = (long long)nx * ny * nz;
     const long long n = npts * nshot;
     const int nzz = nz + 2, nxx = nx + 2;
@@ -274,7 +483,7 @@ __global__ void fsm_crop(const float *__restrict__ T, int NS, float *__restrict_
         const int z = (int)(r % nz);
         const long long r2 = r / nz;
         const int x = (int)(r2 % nx), y = (int)(r2 / nx);
-        out[q] = T[((z + 1) + (long long)(x + 1) * nzz + (long long)(y + 1) * nxx * nzz) * NS + s];
+        out[q] = T[s * nB + (z + 1) + (long long)(x + 1) * nzz + (long long)(y + 1) * nxx * nzz];
     }
 }
 
@@ -297,6 +506,21 @@ static FsmGeo fsm_geo(const st_ctx *ctx) {
     g.dz2dy2 = g.dz2i * g.dy2i;
     g.dx2dy2 = g.dx2i * g.dy2i;
     g.dsum = g.dz2i + g.dx2i + g.dy2i;
+    g.zx = g.dz2i + g.dx2i;
+    g.zy = g.dz2i + g.dy2i;
+    g.xy = g.dx2i + g.dy2i;
+    g.rzx = 1.0f / g.zx;
+    g.rzy = 1.0f / g.zy;
+    g.rxy = 1.0f / g.xy;
+    g.rdsum = 1.0f / g.dsum;
+    g.dmin = 0.99f * std::min({g.dx, g.dy, g.dz});
+    const float z = g.dz2i / g.dsum, x = g.dx2i / g.dsum, y = g.dy2i / g.dsum;
+    g.wv = z - 0.5f * (x + y);
+    g.we = x - 0.5f * (z + y);
+    g.wn = y - 0.5f * (z + x);
+    g.wev = 0.5f * (x + z) - y;
+    g.wen = 0.5f * (x + y) - z;
+    g.wnv = 0.5f * (z + y) - x;
     return g;
 }
 
@@ -305,15 +529,57 @@ static FsmGeo fsm_geo(const st_ctx *ctx) {
 static const int kDirs[8][3] = {{1, 1, 1},  {-1, 1, 1},  {1, 1, -1},  {-1, 1, -1},
                                 {1, -1, 1}, {-1, -1, 1}, {1, -1, -1}, {-1, -1, -1}};
 
-// Shots per device pass are padded to a multiple of 64 (one wave = one cell
-// for 64 shots).
-int fsm_lanes(int nshot) { return (nshot + 63) / 64 * 64; }
+// Whether the FAST update's ranges hold: spacings and their squares far from
+// under- and overflow and within a factor of 1000 of each other (the slack of
+// its 2D bound), root arguments 0 or above 2^-102, times of ordinary size.
+static bool fsm_fast(const st_ctx *ctx, const FsmGeo &g) {
+    const float lo = std::min({g.dx, g.dy, g.dz}), hi = std::max({g.dx, g.dy, g.dz});
+    return lo > 1e-6f && hi < 1e6f && hi < 1000.0f * lo && ctx->smin > 1e-9f && ctx->smax < 1e4f;
+}
+
+// The sixteen sweeps of nshot shots (padded volumes T, source nodes dsid on
+// the device and hsid on the host) on one stream.
+template <int LZ>
+static void fsm_sweeps(hipStream_t st, bool fast, float *T, const float *S, const int *dsid,
+                       const int *hsid, int nshot, const FsmGeo &g) {
+    for (int pass = 0; pass < 2; pass++) {
+        for (int d = 0; d < 8; d++) {
+            const FsmSweep w{kDirs[d][0], kDirs[d][1], kDirs[d][2], pass == 0 ? 1 : 0};
+            // the longest box along each axis
+            int len[3];
+            const int dir[3] = {w.tz, w.tx, w.ty}, n[3] = {g.nzz, g.nxx, g.nyy};
+            for (int ax = 0; ax < 3; ax++) {
+                len[ax] = 0;
+                for (int s = 0; s < (w.init ? nshot : 1); s++) {
+                    int st0, l;
+                    sweep_axis(dir[ax], w.init, n[ax], hsid[3 * s + ax], st0, l);
+                    len[ax] = std::max(len[ax], l);
+                }
+            }
+            const int nA0 = (len[0] + LZ - 1) / LZ;
+            const int zc = (len[0] + nA0 - 1) / nA0;   // chunks of equal length
+            const int nA = (len[0] + zc - 1) / zc, nB = (len[1] + 7) / 8, nC = (len[2] + 7) / 8;
+            for (int D = 0; D < nA + nB + nC - 2; D++) {
+                const int a0 = std::max(0, D - (nB - 1) - (nC - 1)), a1 = std::min(nA - 1, D);
+                const int c0 = std::max(0, D - (nB - 1) - (nA - 1)), c1 = std::min(nC - 1, D);
+                const int na = a1 - a0 + 1, nc = c1 - c0 + 1;
+                const dim3 grid((unsigned)(na * nc * nshot));
+                if (fast)
+                    hipLaunchKernelGGL((fsm_block<LZ, true>), grid, dim3(64), 0, st, T, S, dsid,
+                                       nshot, g, w, zc, D, a0, na, c0);
+                else
+                    hipLaunchKernelGGL((fsm_block<LZ, false>), grid, dim3(64), 0, st, T, S, dsid,
+                                       nshot, g, w, zc, D, a0, na, c0);
+            }
+            ST_HIP(hipGetLastError());
+        }
+    }
+}
 
 // Solves nshot shots (device sources dsrc, host copies hsrc) into ctx->T
-// (padded volume, shot fastest); returns the device time in ms.
+// (one padded volume per shot); returns the device time in ms.
 double fsm_batch(st_ctx *ctx, const float *dsrc, const float *hsrc, int nshot, const float *S) {
     const FsmGeo g = fsm_geo(ctx);
-    const int NS = fsm_lanes(nshot);
     std::vector<int> hsid(3 * nshot);
     for (int s = 0; s < nshot; s++) {
         hsid[3 * s] = (int)(hsrc[3 * s + 2] / ctx->dz) + 1;      // z
@@ -325,45 +591,15 @@ double fsm_batch(st_ctx *ctx, const float *dsrc, const float *hsrc, int nshot, c
     ST_HIP(hipMemcpyAsync(dsid, hsid.data(), sizeof(int) * 3 * nshot, hipMemcpyHostToDevice,
                           ctx->stream));
     ST_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
-    const long long nT = (long long)NS * g.nB;
+    const long long nT = (long long)nshot * g.nB;
     float *T = ctx->T.as<float>();
     ST_REQUIRE(ctx->T.bytes >= sizeof(float) * (size_t)nT, ST_ERR_STATE, "travel-time buffer too small");
     hipLaunchKernelGGL(fsm_fill, dim3(grid_for(nT / 4)), dim3(256), 0, ctx->stream, T, nT);
-    hipLaunchKernelGGL(fsm_seed, dim3((nshot + 63) / 64), dim3(64), 0, ctx->stream, T, NS, S, dsrc,
+    hipLaunchKernelGGL(fsm_seed, dim3((nshot + 63) / 64), dim3(64), 0, ctx->stream, T, S, dsrc,
                        dsid, nshot, g);
     ST_HIP(hipGetLastError());
-    for (int pass = 0; pass < 2; pass++) {
-        for (int d = 0; d < 8; d++) {
-            const FsmSweep w{kDirs[d][0], kDirs[d][1], kDirs[d][2], pass == 0 ? 1 : 0};
-            // union of the shots' boxes: the earliest start along each direction
-            int start[3], len[3];
-            const int dir[3] = {w.tz, w.tx, w.ty}, n[3] = {g.nzz, g.nxx, g.nyy};
-            for (int ax = 0; ax < 3; ax++) {
-                int best = dir[ax] > 0 ? n[ax] : -1;
-                for (int s = 0; s < nshot; s++) {
-                    int st0, l;
-                    sweep_axis(dir[ax], w.init, n[ax], hsid[3 * s + ax], st0, l);
-                    best = dir[ax] > 0 ? std::min(best, st0) : std::max(best, st0);
-                }
-                start[ax] = best;
-                len[ax] = dir[ax] > 0 ? n[ax] - best : best + 1;
-            }
-            const int zl = len[0], xl = len[1], yl = len[2];
-            const int P = zl + xl + yl - 2;
-            for (int p = 0; p < P; p++) {
-                // a in [p - (xl-1) - (yl-1), p] cap [0, zl); c likewise
-                const int a0 = std::max(0, p - (xl - 1) - (yl - 1)), a1 = std::min(zl - 1, p);
-                const int c0 = std::max(0, p - (xl - 1) - (zl - 1)), c1 = std::min(yl - 1, p);
-                if (a1 < a0 || c1 < c0) continue;
-                const int na = a1 - a0 + 1, nc = c1 - c0 + 1;
-                const long long nt = (long long)na * nc * NS;
-                hipLaunchKernelGGL(fsm_plane, dim3((unsigned)((nt + 255) / 256)), dim3(256), 0,
-                                   ctx->stream, T, NS, nshot, S, dsid, g, w, start[0], start[1],
-                                   start[2], xl, p, a0, na, c0, nc);
-            }
-            ST_HIP(hipGetLastError());
-        }
-    }
+    const bool fast = fsm_fast(ctx, g);
+    fsm_sweeps<kFsmZ>(ctx->stream, fast, T, S, dsid, hsid.data(), nshot, g);
     ST_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
     ST_HIP(hipEventSynchronize(ctx->ev[3]));
     float ms = 0.f;
@@ -379,14 +615,14 @@ void fsm_pad(st_ctx *ctx, float *S) {
 }
 
 void fsm_picks(st_ctx *ctx, int nshot, const float *drcv, int nrcv, float *dpicks) {
-    launch_picks_pad(ctx->stream, ctx->T.as<float>(), fsm_lanes(nshot), nshot, drcv, nrcv, dpicks,
-                     ctx->nx, ctx->ny, ctx->nz, ctx->dx, ctx->dy, ctx->dz);
+    launch_picks_padvol(ctx->stream, ctx->T.as<float>(), fsm_geo(ctx).nB, nshot, drcv, nrcv,
+                        dpicks, ctx->nx, ctx->ny, ctx->nz, ctx->dx, ctx->dy, ctx->dz);
 }
 
 void fsm_crop_volumes(st_ctx *ctx, float *dout, int nshot) {
     const long long n = (long long)ctx->nx * ctx->ny * ctx->nz * nshot;
     hipLaunchKernelGGL(fsm_crop, dim3(grid_for(n)), dim3(256), 0, ctx->stream, ctx->T.as<float>(),
-                       fsm_lanes(nshot), dout, ctx->nx, ctx->ny, ctx->nz, nshot);
+                       dout, ctx->nx, ctx->ny, ctx->nz, fsm_geo(ctx).nB, nshot);
     ST_HIP(hipGetLastError());
 }
 

@@ -107,13 +107,11 @@ struct ZxyLay {
     }
 };
 // the sweeping solvers' volumes, padded by one cell on every side (the
-// reference's expand_fdm extent); cells are cs floats apart (Accurate_FSM
-// keeps the shots of a batch fastest, cs = its shot lanes; Podvin cs = 1)
+// reference's expand_fdm extent), z fastest
 struct PadLay {
-    int nxx, nzz, cs;
+    int nxx, nzz;
     __device__ long long operator()(int x, int y, int z) const {
-        return ((long long)(z + 1) + (long long)(x + 1) * nzz + (long long)(y + 1) * nxx * nzz) *
-               cs;
+        return (long long)(z + 1) + (long long)(x + 1) * nzz + (long long)(y + 1) * nxx * nzz;
     }
 };
 // solver block layout for a power-of-two block edge 1 << lb and in-volume
@@ -130,21 +128,6 @@ struct BlkLay {
                (((unsigned)z & m) << (2 * lb));
     }
 };
-
-// RN(a / b) for b > 0 from y = RN(1 / b) without a division: q = a y, one
-// fma residual correction makes q faithful, and Markstein's final step (the
-// residual a - b q is exact by fma, q + r y rounded once) returns the
-// correctly rounded quotient.  Where intermediate results could leave the
-// normal range (|a / b| < 2^-100), the quotient's integer part, the only use
-// here, is 0 either way.  Checked against IEEE division on every float
-// |a| in [2^-20, 2^20) for 16 spacings from 1e-3 to 9999: all bits equal.
-__device__ __forceinline__ float div_rn(float a, float b, float y) {
-    float q = a * y;
-    float r = __builtin_fmaf(-q, b, a);
-    q = __builtin_fmaf(r, y, q);
-    r = __builtin_fmaf(-q, b, a);
-    return __builtin_fmaf(r, y, q);
-}
 
 struct RayArgs {
     const float *T;
@@ -1446,10 +1429,10 @@ void tomo_model_update(st_ctx *ctx, const float *dxdm, int smooth, int samples, 
     model_changed(ctx);  // derived copies of the slowness are rebuilt on the next solve
 }
 
-void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, int cell_stride,
-                    const float *dsrc, int nshot, const float *drcv, int nr, bool with_illum) {
-    trace_append(ctx, T, shot_stride, PadLay{ctx->nx + 2, ctx->nz + 2, cell_stride}, dsrc, nshot,
-                 drcv, nr, with_illum);
+void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, const float *dsrc,
+                    int nshot, const float *drcv, int nr, bool with_illum) {
+    trace_append(ctx, T, shot_stride, PadLay{ctx->nx + 2, ctx->nz + 2}, dsrc, nshot, drcv, nr,
+                 with_illum);
 }
 
 void tomo_trace_zxy(st_ctx *ctx, const float *dT, const float *dsrc, const float *drcv, int nr,
