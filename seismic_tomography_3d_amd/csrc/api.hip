@@ -37,12 +37,12 @@ void tomo_release(st_ctx *ctx);
 void surrogate_release(st_ctx *ctx);
 void wave_release(st_ctx *ctx);
 size_t podvin_bytes_per_shot(const st_ctx *ctx);
-double podvin_batch(st_ctx *ctx, const float *dsrc, const float *hsrc, int nshot, const float *S,
-                    float *T, int *stamp, int *list, float *newv, int *count, int *nit_dev,
-                    DevBuf &temp);
-void podvin_picks(st_ctx *ctx, const float *T, int nshot, const float *drcv, int nrcv,
-                  float *dpicks);
-void podvin_crop_volumes(st_ctx *ctx, const float *T, float *dout, int nshot);
+void podvin_layout(const st_ctx *ctx, long long &stride, int &nxx, int &nzz);
+long long podvin_max_batch(const st_ctx *ctx);
+void podvin_reserve(st_ctx *ctx, int batch);
+double podvin_batch(st_ctx *ctx, const float *dsrc, const float *hsrc, int nshot);
+void podvin_picks(st_ctx *ctx, int nshot, const float *drcv, int nrcv, float *dpicks);
+void podvin_crop_volumes(st_ctx *ctx, float *dout, int nshot);
 void acoustic_dampers(float *d1, float *d2, float *d3, float factor, int nb);
 void acoustic_ricker(float delay, float fmax, float dt, int nt, float *out);
 void wave_set_model(st_ctx *ctx, const float *vel, int nx, int ny, int nz, float dx, float dy,
@@ -61,8 +61,8 @@ void tomo_trace_blk(st_ctx *ctx, const float *T, long long vol, int B, int nbx, 
                     const float *dsrc, int nshot, const float *drcv, int nr, bool with_illum);
 void tomo_trace_zxy(st_ctx *ctx, const float *dT, const float *dsrc, const float *drcv, int nr,
                     bool with_illum);
-void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, const float *dsrc,
-                    int nshot, const float *drcv, int nr, bool with_illum);
+void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, int nxx, int nzz,
+                    const float *dsrc, int nshot, const float *drcv, int nr, bool with_illum);
 void tomo_get_illum(st_ctx *ctx, float *out);
 void tomo_csr(st_ctx *ctx, long long *rows, long long *nnz, const long long **rp, const int **c,
               const float **v);
@@ -266,7 +266,7 @@ int st_ctx_destroy(st_ctx *ctx) {
     for (auto *b : {&ctx->slow_zxy, &ctx->range, &ctx->slow_blk[0], &ctx->slow_blk[1], &ctx->T, &ctx->flags,
                     &ctx->list[0], &ctx->list[1], &ctx->counters, &ctx->wstats, &ctx->fsm_S,
                     &ctx->fsm_sid, &ctx->pod_T, &ctx->pod_stamp, &ctx->pod_list,
-                    &ctx->pod_newv, &ctx->pod_counts, &ctx->pod_nit, &ctx->pod_temp,
+                    &ctx->pod_counts, &ctx->pod_nit,
                     &ctx->src, &ctx->rcv,
                     &ctx->picks, &ctx->scratch, &ctx->keys, &ctx->kmin, &ctx->judge, &ctx->pred,
                     &ctx->tkeys, &ctx->xfaces})
@@ -355,41 +355,20 @@ static int fsm_setup(st_ctx *ctx, int nshot, int batch, bool with_T_out) {
     return b;
 }
 
-// Podvin's padded slowness (the sweeping solver's one-cell replicated pad)
-// and per-shot buffers; returns the batch size (batch <= 0: 16).
+// Podvin's per-shot buffers; returns the batch size (batch <= 0: 16).
 static int podvin_setup(st_ctx *ctx, int nshot, int batch, bool with_T_out) {
-    const long long nB = (long long)(ctx->nx + 2) * (ctx->ny + 2) * (ctx->nz + 2);
     const long long npts = (long long)ctx->nx * ctx->ny * ctx->nz;
-    if (!ctx->fsm_valid) {
-        ctx->fsm_S.reserve(sizeof(float) * nB);
-        fsm_pad(ctx, ctx->fsm_S.as<float>());
-        ctx->fsm_valid = true;
-    }
     int b = batch > 0 ? std::min(batch, nshot) : std::min(nshot, 16);
-    // list items and counts are 32-bit: shots x padded cells below 2^31
-    while (b > 1 && (long long)b * nB >= (1LL << 31)) b /= 2;
+    b = (int)std::max(1LL, std::min<long long>(b, podvin_max_batch(ctx)));
     size_t free_b = 0, total_b = 0;
     ST_HIP(hipMemGetInfo(&free_b, &total_b));
     const size_t per_shot = podvin_bytes_per_shot(ctx) + (with_T_out ? sizeof(float) * npts : 0);
     const size_t have = free_b + ctx->pod_T.bytes + ctx->pod_stamp.bytes + ctx->pod_list.bytes +
-                        ctx->pod_newv.bytes + ctx->scratch.bytes;
+                        ctx->scratch.bytes;
     while (b > 1 && per_shot * (size_t)b > have / 2) b /= 2;
-    ctx->pod_T.reserve(sizeof(float) * nB * b);
-    ctx->pod_stamp.reserve(sizeof(int) * nB * b);
-    ctx->pod_list.reserve(sizeof(int) * nB * b);
-    ctx->pod_newv.reserve(sizeof(float) * nB * b);
-    ctx->pod_counts.reserve(sizeof(int) * 64);
-    ctx->pod_nit.reserve(sizeof(int) * b);
+    podvin_reserve(ctx, b);
     if (with_T_out) ctx->scratch.reserve(sizeof(float) * npts * b);
     return b;
-}
-
-// Podvin over shots b0 .. b0 + nb - 1 of the uploaded sources into pod_T.
-static double podvin_run(st_ctx *ctx, int b0, int nb, const float *src_xyz) {
-    return podvin_batch(ctx, ctx->src.as<float>() + 3LL * b0, src_xyz + 3LL * b0, nb,
-                        ctx->fsm_S.as<float>(), ctx->pod_T.as<float>(), ctx->pod_stamp.as<int>(),
-                        ctx->pod_list.as<int>(), ctx->pod_newv.as<float>(),
-                        ctx->pod_counts.as<int>(), ctx->pod_nit.as<int>(), ctx->pod_temp);
 }
 
 static void solve_impl(st_ctx *ctx, const float *src_xyz, int nshot, const float *rcv_xyz,
@@ -720,12 +699,12 @@ int st_podvin_solve(st_ctx *ctx, const float *src_xyz, int nshot, const float *r
         double ms = 0.0;
         for (int b0 = 0; b0 < nshot; b0 += b) {
             const int nb = std::min(b, nshot - b0);
-            ms += podvin_run(ctx, b0, nb, src_xyz);
+            ms += podvin_batch(ctx, ctx->src.as<float>() + 3LL * b0, src_xyz + 3LL * b0, nb);
             if (nrcv)
-                podvin_picks(ctx, ctx->pod_T.as<float>(), nb, ctx->rcv.as<float>(), nrcv,
+                podvin_picks(ctx, nb, ctx->rcv.as<float>(), nrcv,
                              ctx->picks.as<float>() + (long long)b0 * nrcv);
             if (T_out) {
-                podvin_crop_volumes(ctx, ctx->pod_T.as<float>(), ctx->scratch.as<float>(), nb);
+                podvin_crop_volumes(ctx, ctx->scratch.as<float>(), nb);
                 ST_HIP(hipMemcpyAsync(T_out + (long long)b0 * npts, ctx->scratch.ptr,
                                       sizeof(float) * npts * nb, hipMemcpyDeviceToHost,
                                       ctx->stream));
@@ -905,7 +884,8 @@ static void forward_impl(st_ctx *ctx, const float *src_xyz, int nshot, const flo
             const double t = fsm_batch(ctx, dsrc, src_xyz + 3LL * b0, nb, ctx->fsm_S.as<float>());
             if (stats) { stats->solve_ms += t; stats->batches += 1; }
             fsm_picks(ctx, nb, drcv, nrcv, ctx->picks.as<float>() + (long long)b0 * nrcv);
-            tomo_trace_pad(ctx, ctx->T.as<float>(), nB, dsrc, nb, drcv, nrcv, true);
+            tomo_trace_pad(ctx, ctx->T.as<float>(), nB, ctx->nx + 2, ctx->nz + 2, dsrc, nb, drcv, nrcv,
+                           true);
             if (T_out) {
                 fsm_crop_volumes(ctx, ctx->scratch.as<float>(), nb);
                 to_host(b0, nb);
@@ -914,17 +894,18 @@ static void forward_impl(st_ctx *ctx, const float *src_xyz, int nshot, const flo
     } else {
         // Podvin & Lecomte: shot-major padded volumes
         const int b = podvin_setup(ctx, nshot, 0, T_out != nullptr);
-        const long long nB = (long long)(ctx->nx + 2) * (ctx->ny + 2) * (ctx->nz + 2);
+        long long stride;
+        int nxx, nzz;
+        podvin_layout(ctx, stride, nxx, nzz);
         for (int b0 = 0; b0 < nshot; b0 += b) {
             const int nb = std::min(b, nshot - b0);
             const float *dsrc = ctx->src.as<float>() + 3LL * b0;
-            const double t = podvin_run(ctx, b0, nb, src_xyz);
+            const double t = podvin_batch(ctx, dsrc, src_xyz + 3LL * b0, nb);
             if (stats) { stats->solve_ms += t; stats->batches += 1; }
-            podvin_picks(ctx, ctx->pod_T.as<float>(), nb, drcv, nrcv,
-                         ctx->picks.as<float>() + (long long)b0 * nrcv);
-            tomo_trace_pad(ctx, ctx->pod_T.as<float>(), nB, dsrc, nb, drcv, nrcv, true);
+            podvin_picks(ctx, nb, drcv, nrcv, ctx->picks.as<float>() + (long long)b0 * nrcv);
+            tomo_trace_pad(ctx, ctx->pod_T.as<float>(), stride, nxx, nzz, dsrc, nb, drcv, nrcv, true);
             if (T_out) {
-                podvin_crop_volumes(ctx, ctx->pod_T.as<float>(), ctx->scratch.as<float>(), nb);
+                podvin_crop_volumes(ctx, ctx->scratch.as<float>(), nb);
                 to_host(b0, nb);
             }
         }

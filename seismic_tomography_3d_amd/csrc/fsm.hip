@@ -46,9 +46,9 @@
 
 namespace st {
 
-void launch_picks_padvol(hipStream_t st, const float *T, long long vol, int nshot,
-                         const float *rcv, int nr, float *out, int nx, int ny, int nz, float dx,
-                         float dy, float dz);
+void launch_picks_padvol(hipStream_t st, const float *T, long long vol, int nxx, int nzz,
+                         int nshot, const float *rcv, int nr, float *out, int nx, int ny, int nz,
+                         float dx, float dy, float dz);
 
 __device__ __forceinline__ float smin(float a, float b) { return (b < a) ? b : a; }
 __device__ __forceinline__ float smax(float a, float b) { return (a < b) ? b : a; }
@@ -615,7 +615,8 @@ void fsm_pad(st_ctx *ctx, float *S) {
 }
 
 void fsm_picks(st_ctx *ctx, int nshot, const float *drcv, int nrcv, float *dpicks) {
-    launch_picks_padvol(ctx->stream, ctx->T.as<float>(), fsm_geo(ctx).nB, nshot, drcv, nrcv,
+    const FsmGeo g = fsm_geo(ctx);
+    launch_picks_padvol(ctx->stream, ctx->T.as<float>(), g.nB, g.nxx, g.nzz, nshot, drcv, nrcv,
                         dpicks, ctx->nx, ctx->ny, ctx->nz, ctx->dx, ctx->dy, ctx->dz);
 }
 

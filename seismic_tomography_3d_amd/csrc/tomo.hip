@@ -1429,10 +1429,9 @@ void tomo_model_update(st_ctx *ctx, const float *dxdm, int smooth, int samples, 
     model_changed(ctx);  // derived copies of the slowness are rebuilt on the next solve
 }
 
-void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, const float *dsrc,
-                    int nshot, const float *drcv, int nr, bool with_illum) {
-    trace_append(ctx, T, shot_stride, PadLay{ctx->nx + 2, ctx->nz + 2}, dsrc, nshot, drcv, nr,
-                 with_illum);
+void tomo_trace_pad(st_ctx *ctx, const float *T, long long shot_stride, int nxx, int nzz,
+                    const float *dsrc, int nshot, const float *drcv, int nr, bool with_illum) {
+    trace_append(ctx, T, shot_stride, PadLay{nxx, nzz}, dsrc, nshot, drcv, nr, with_illum);
 }
 
 void tomo_trace_zxy(st_ctx *ctx, const float *dT, const float *dsrc, const float *drcv, int nr,
