@@ -574,6 +574,7 @@ int st_fim_solve_noalloc(st_ctx *ctx, const float *src_xyz, int nshot, const flo
             f.list0 = c.take<unsigned>(fim_list_bytes(g.nblk, b) / sizeof(unsigned));
             f.list1 = c.take<unsigned>(fim_list_bytes(g.nblk, b) / sizeof(unsigned));
             f.kmin = tentative ? c.take<unsigned>(3 * (size_t)b) : nullptr;
+            f.kstride = b;
             f.tk = tentative ? c.take<unsigned>(2 * (size_t)b * g.nblk) : nullptr;
             f.wstats = stats ? c.take<unsigned long long>(3 * (size_t)nwaves) : nullptr;
             f.xf = B == 8 ? c.take<float>(128 * (size_t)b * g.nblk) : nullptr;

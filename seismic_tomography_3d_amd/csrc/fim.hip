@@ -56,7 +56,12 @@ struct FimArgs {
     // key exceeds (smallest key of its shot's current list + band) is
     // deferred to the next round instead of visited
     const float *keys;         // per (shot, block) predicted first arrival
-    unsigned *kmin;            // [3][nshot] per-shot smallest key of each list (float bits)
+    // per-shot smallest key of each list (float bits), [3][ksub][kstride]: a
+    // shot's minimum is the least of its ksub words (a power of two), each on a
+    // line of its own and lowered by every ksub-th wave, since a round's waves
+    // would otherwise queue for one line
+    unsigned *kmin;
+    int ksub, kstride;
     int nshot;
     float band;
     const float *src;          // the batch's sources, 3 per shot (x, y, z in m)
@@ -122,56 +127,6 @@ __device__ __forceinline__ float godunov(float a, float b, float c, float hs, fl
     return r > hi ? t3 : r;
 }
 
-// Schedules the candidates held by lanes 0..6 for the next round and
-// appends the newly scheduled ones to the next list.
-__device__ __forceinline__ void schedule(const FimArgs &A, unsigned shot, unsigned *fl,
-                                         unsigned target, unsigned bit_nxt, unsigned *nxt,
-                                         unsigned *nxt_cnt, int lane, float key) {
-    bool fresh = false, claim = false;
-    if (target != 0xFFFFFFFFu) {
-        const unsigned old = atomicOr(&fl[target], bit_nxt | (A.lazy ? 4u : 0u));
-        fresh = !(old & bit_nxt);
-        claim = A.lazy && !(old & 4u);
-        // the claim's stamp (one writer, so an OR)
-        if (claim) atomicOr(&fl[target], ((unsigned)A.epoch + 2u) << 3);
-        if (A.tk) {
-            // every scheduler lowers the next list's key (the item itself is
-            // appended once, by the first); with predictions too, the block
-            // counts as due no earlier than its predicted arrival
-            atomicMin(&A.tk[((long long)((A.round + 1) & 1) * A.nshot + shot) * A.nblk + target],
-                      __float_as_uint(key));
-            const float eff = A.keys ? fmaxf(key, A.keys[(long long)shot * A.nblk + target]) : key;
-            atomicMin(&A.kmin[((A.round + 1) % 3) * A.nshot + shot], __float_as_uint(eff));
-        } else if (fresh && A.keys) {
-            atomicMin(&A.kmin[((A.round + 1) % 3) * A.nshot + shot],
-                      __float_as_uint(A.keys[(long long)shot * A.nblk + target]));
-        }
-    }
-    const unsigned long long fm = __ballot(fresh);
-    if (fm) {
-        unsigned base = 0;
-        if (lane == 0) base = atomicAdd(nxt_cnt, (unsigned)__popcll(fm));
-        base = (unsigned)__builtin_amdgcn_readlane((int)base, 0);
-        if (fresh) {
-            const unsigned rank = (unsigned)__popcll(fm & ((1ull << lane) - 1ull));
-            nxt[base + rank] = (shot << kShotShift) | target;
-        }
-    }
-    // claimed blocks' cold fill, by the whole wave: 512 cells, 128 face values
-    unsigned long long cm = __ballot(claim);
-    while (cm) {
-        const int j = __builtin_ctzll(cm);
-        cm &= cm - 1ull;
-        const long long tb = (long long)(unsigned)__builtin_amdgcn_readlane((int)target, j);
-        float4 *p = reinterpret_cast<float4 *>(A.T + (long long)shot * A.vol + tb * 512);
-        p[lane] = make_float4(kInf, kInf, kInf, kInf);
-        p[lane + 64] = make_float4(kInf, kInf, kInf, kInf);
-        if (A.xf)
-            reinterpret_cast<float2 *>(A.xf + ((long long)shot * A.nblk + tb) * 128)[lane] =
-                make_float2(kInf, kInf);
-    }
-}
-
 // Minimum over the lanes whose index differs from this lane's only in the
 // bits of mask (a butterfly over those bits).
 // Cross-lane minima in the VALU (DPP), without LDS permutes: a DPP move
@@ -223,6 +178,69 @@ __device__ __forceinline__ float wave_max_all(float v) {
     return fmaxf(fmaxf(lane_val(v, 0), lane_val(v, 16)), fmaxf(lane_val(v, 32), lane_val(v, 48)));
 }
 
+constexpr int kKeySub = 8;   // most words per shot's smallest key (a power of two)
+
+// Sub-word `sub` of a shot's smallest key of the list in slot (round mod 3).
+__device__ __forceinline__ unsigned *kmin_at(const FimArgs &A, int round, unsigned sub,
+                                             unsigned shot) {
+    return A.kmin + ((round % 3) * A.ksub + (sub & (A.ksub - 1))) * A.kstride + shot;
+}
+
+// Schedules the candidates held by lanes 0..6 for the next round and
+// appends the newly scheduled ones to the next list.
+template <int KM>
+__device__ __forceinline__ void schedule(const FimArgs &A, unsigned shot, unsigned *fl,
+                                         unsigned target, unsigned bit_nxt, unsigned *nxt,
+                                         unsigned *nxt_cnt, int lane, unsigned gw, float key) {
+    bool fresh = false, claim = false;
+    float eff = __builtin_inff();
+    if (target != 0xFFFFFFFFu) {
+        const unsigned old = atomicOr(&fl[target], bit_nxt | (A.lazy ? 4u : 0u));
+        fresh = !(old & bit_nxt);
+        claim = A.lazy && !(old & 4u);
+        // the claim's stamp (one writer, so an OR)
+        if (claim) atomicOr(&fl[target], ((unsigned)A.epoch + 2u) << 3);
+        if constexpr (KM & 1) {
+            // every scheduler lowers the next list's key (the item itself is
+            // appended once, by the first); with predictions too, the block
+            // counts as due no earlier than its predicted arrival
+            atomicMin(&A.tk[((long long)((A.round + 1) & 1) * A.nshot + shot) * A.nblk + target],
+                      __float_as_uint(key));
+            eff = key;
+            if constexpr (KM & 2) eff = fmaxf(key, A.keys[(long long)shot * A.nblk + target]);
+        } else if constexpr (KM & 2) {
+            if (fresh) eff = A.keys[(long long)shot * A.nblk + target];
+        }
+    }
+    if constexpr (KM) {   // the targets are in lanes 0..6: one atomic for the wave
+        const unsigned m = __float_as_uint(min8(eff));
+        if (lane == 0 && m != kInfBits) atomicMin(kmin_at(A, A.round + 1, gw >> 4, shot), m);
+    }
+    const unsigned long long fm = __ballot(fresh);
+    if (fm) {
+        unsigned base = 0;
+        if (lane == 0) base = atomicAdd(nxt_cnt, (unsigned)__popcll(fm));
+        base = (unsigned)__builtin_amdgcn_readlane((int)base, 0);
+        if (fresh) {
+            const unsigned rank = (unsigned)__popcll(fm & ((1ull << lane) - 1ull));
+            nxt[base + rank] = (shot << kShotShift) | target;
+        }
+    }
+    // claimed blocks' cold fill, by the whole wave: 512 cells, 128 face values
+    unsigned long long cm = __ballot(claim);
+    while (cm) {
+        const int j = __builtin_ctzll(cm);
+        cm &= cm - 1ull;
+        const long long tb = (long long)(unsigned)__builtin_amdgcn_readlane((int)target, j);
+        float4 *p = reinterpret_cast<float4 *>(A.T + (long long)shot * A.vol + tb * 512);
+        p[lane] = make_float4(kInf, kInf, kInf, kInf);
+        p[lane + 64] = make_float4(kInf, kInf, kInf, kInf);
+        if (A.xf)
+            reinterpret_cast<float2 *>(A.xf + ((long long)shot * A.nblk + tb) * 128)[lane] =
+                make_float2(kInf, kInf);
+    }
+}
+
 template <int MASK>
 __device__ __forceinline__ float lane_min(float v) {
 #pragma unroll
@@ -263,7 +281,7 @@ __device__ __forceinline__ void round_counts(const FimArgs &A, int lane, unsigne
 // due yet (predicted arrival above its shot's earliest scheduled key plus
 // the band) move to the next list right here, all lanes at once with one
 // append; the others are visited one after another by the whole wave.
-template <class Visit>
+template <int KM, class Visit>
 __device__ __forceinline__ void for_items(const FimArgs &A, unsigned count, unsigned incl,
                                           const unsigned *cur, unsigned *nxt, unsigned *nxt_cnt,
                                           unsigned bit_cur, unsigned bit_nxt, int lane,
@@ -275,6 +293,9 @@ __device__ __forceinline__ void for_items(const FimArgs &A, unsigned count, unsi
         // flat index -> (segment, offset): incl holds, in lane k < kSeg, the
         // inclusive prefix of the segment lengths
         unsigned seg = 0, before = 0;
+        // (opaque: the segment bounds read from incl are the same in every
+        // turn of this loop and would be kept in scalar registers throughout)
+        asm volatile("" : "+v"(incl));
 #pragma unroll
         for (int k = 0; k < kSeg - 1; k++) {
             const unsigned ik = (unsigned)__builtin_amdgcn_readlane((int)incl, k);
@@ -282,22 +303,30 @@ __device__ __forceinline__ void for_items(const FimArgs &A, unsigned count, unsi
         }
         const unsigned item = in ? cur[seg * A.cap + (i - before)] : 0u;
         bool run = in;
-        if (A.keys || A.tk) {
+        if constexpr (KM) {
             bool fresh = false;
             unsigned shot = 0;
             if (in) {
                 shot = item >> kShotShift;
                 const unsigned b = item & kBlkMask;
-                const float tau =
-                    __uint_as_float(A.kmin[(A.round % 3) * A.nshot + shot]) + A.band;
+                unsigned km = *kmin_at(A, A.round, 0, shot);
+                if (A.ksub > 1) {   // loads in flight together (indices wrap)
+                    unsigned w[kKeySub - 1];
+#pragma unroll
+                    for (int k = 1; k < kKeySub; k++) w[k - 1] = *kmin_at(A, A.round, k, shot);
+#pragma unroll
+                    for (int k = 1; k < kKeySub; k++) km = min(km, w[k - 1]);
+                }
+                const float tau = __uint_as_float(km) + A.band;
                 float key, kt = 0.0f;
-                if (A.tk) {
+                if constexpr (KM & 1) {
                     // this list's key is consumed here (visited or carried
                     // over); only the next list's keys are written this round
                     unsigned *kc = A.tk + ((long long)(A.round & 1) * A.nshot + shot) * A.nblk + b;
                     kt = __uint_as_float(*kc);
                     *kc = kInfBits;
-                    key = A.keys ? fmaxf(kt, A.keys[(long long)shot * A.nblk + b]) : kt;
+                    key = kt;
+                    if constexpr (KM & 2) key = fmaxf(kt, A.keys[(long long)shot * A.nblk + b]);
                 } else {
                     key = A.keys[(long long)shot * A.nblk + b];
                 }
@@ -306,13 +335,12 @@ __device__ __forceinline__ void for_items(const FimArgs &A, unsigned count, unsi
                     unsigned *fl = A.flags + (long long)shot * A.nblk;
                     atomicAnd(&fl[b], ~bit_cur);
                     fresh = !(atomicOr(&fl[b], bit_nxt) & bit_nxt);
-                    if (A.tk) {
+                    if constexpr (KM & 1) {
                         atomicMin(&A.tk[((long long)((A.round + 1) & 1) * A.nshot + shot) * A.nblk + b],
                                   __float_as_uint(kt));
-                        atomicMin(&A.kmin[((A.round + 1) % 3) * A.nshot + shot], __float_as_uint(key));
+                        atomicMin(kmin_at(A, A.round + 1, gw >> 4, shot), __float_as_uint(key));
                     } else if (fresh) {
-                        atomicMin(&A.kmin[((A.round + 1) % 3) * A.nshot + shot],
-                                  __float_as_uint(key));
+                        atomicMin(kmin_at(A, A.round + 1, gw >> 4, shot), __float_as_uint(key));
                     }
                 }
             }
@@ -337,19 +365,22 @@ __device__ __forceinline__ void for_items(const FimArgs &A, unsigned count, unsi
 // ---------------------------------------------------------------------------
 // 4^3 blocks: lane = tx + 4 ty + 16 tz, one cell per lane, Jacobi sweeps.
 // ---------------------------------------------------------------------------
+template <int KM>
 __global__ __launch_bounds__(64 * kWaves) void fim_round4(FimArgs A) {
     __shared__ float tiles[kWaves][216];  // (4+2)^3, index x + 6 y + 36 z
     const int lane = threadIdx.x & 63;
-    float *tile = tiles[threadIdx.x >> 6];
-    const unsigned gw = blockIdx.x * kWaves + (threadIdx.x >> 6), G = gridDim.x * kWaves;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // this wave (scalar)
+    float *tile = tiles[wv];
+    const unsigned gw = blockIdx.x * kWaves + wv, G = gridDim.x * kWaves;
     const int p = A.round & 1;
     unsigned incl = 0, count = 0;
     round_counts(A, lane, incl, count);
     if (gw == 0) {
         if (lane < kSeg) A.cnt[(((A.round + 2) % 3) * kSeg + lane) * kCntStride] = 0;
         if (lane == 0 && count) atomicAdd(&A.cnt[kRoundsIdx], 1u);
-        if (A.keys || A.tk)
-            for (int j = lane; j < A.nshot; j += 64) A.kmin[((A.round + 2) % 3) * A.nshot + j] = kInfBits;
+        if constexpr (KM)
+            for (int j = lane; j < A.ksub * A.kstride; j += 64)
+                A.kmin[((A.round + 2) % 3) * A.ksub * A.kstride + j] = kInfBits;
     }
     if (count == 0) return;
     const unsigned *cur = p ? A.list1 : A.list0;
@@ -364,7 +395,7 @@ __global__ __launch_bounds__(64 * kWaves) void fim_round4(FimArgs A) {
     const int nbxy = A.nbx * A.nby;
     unsigned long long my_visits = 0, my_iters = 0, my_defer = 0;
 
-    for_items(A, count, incl, cur, nxt, nxt_cnt, bit_cur, bit_nxt, lane, gw, G, my_defer, [&](const unsigned item) {
+    for_items<KM>(A, count, incl, cur, nxt, nxt_cnt, bit_cur, bit_nxt, lane, gw, G, my_defer, [&](const unsigned item) {
         const unsigned shot = item >> kShotShift, b = item & kBlkMask;
         float *Tsh = A.T + (long long)shot * A.vol;
         unsigned *fl = A.flags + (long long)shot * A.nblk;
@@ -443,7 +474,7 @@ __global__ __launch_bounds__(64 * kWaves) void fim_round4(FimArgs A) {
         default: break;
         }
         float key = kKeyInf;
-        if (A.tk) {
+        if constexpr (KM & 1) {
             // per face, the smallest new value among the cells that activate
             // the neighbour; for a self-reschedule, among the changed cells
             auto face = [&](bool c) { return lane_min<63>(c ? v : kKeyInf); };
@@ -456,7 +487,7 @@ __global__ __launch_bounds__(64 * kWaves) void fim_round4(FimArgs A) {
             key = lane == 0 ? k0 : lane == 1 ? k1 : lane == 2 ? k2 : lane == 3 ? k3
                 : lane == 4 ? k4 : lane == 5 ? k5 : k6;
         }
-        schedule(A, shot, fl, target, bit_nxt, nxt, nxt_cnt, lane, key);
+        schedule<KM>(A, shot, fl, target, bit_nxt, nxt, nxt_cnt, lane, gw, key);
         my_visits += 1;
         my_iters += it;
         wave_sync();
@@ -482,8 +513,14 @@ __global__ __launch_bounds__(64 * kWaves) void fim_round4(FimArgs A) {
 // in that octant is carried through it in one pass; the z sweeps then
 // confirm or finish the fixed point.
 // ---------------------------------------------------------------------------
-// Six waves per SIMD (80 VGPRs, a few spilled values outside the plane
-// loops) measured 10 % faster than five without spills.
+// Six waves per SIMD measured 10 % faster than five and 4 % faster than seven
+// (which spills).  The kernel is bound by vector issue, so what the compiler
+// adds counts: KM, the keys in use (bit 0 the solve's own arrivals, bit 1
+// predictions), is a template argument, the wave's index and pointers are
+// scalar (74 to 78 VGPRs), and the arrival keys of a visit go through values
+// instead of masks held side by side, whose spilled scalar registers had cost
+// a tenth of its instructions.  256 shots of 201 x 201 x 101: unordered 21.7 ->
+// 20.6 ms, in arrival order 17.9 -> 16.8, ordered by the network 20.7 -> 20.2.
 //
 // Tile layout: cell (x, y, z) of the (8+2)^3 tile (halo at 0 and 9) at word
 // x + 104 y + 10 z - 11.  gfx950's LDS serves a wave64 access from 64 banks:
@@ -502,22 +539,24 @@ __host__ __device__ __forceinline__ constexpr int tix(int x, int y, int z) {
 constexpr int kTile8 = tix(8, 9, 8) + 1;
 static_assert(tix(1, 0, 1) == 0 && tix(0, 1, 1) > 0 && tix(1, 1, 0) > 0, "tile base");
 static_assert(tix(9, 8, 8) < kTile8 && tix(8, 8, 9) < kTile8 && kTile8 == 1014, "tile span");
-template <bool HYP>
+template <bool HYP, int KM>
 __global__ __launch_bounds__(64 * kWaves, 6) void fim_round8(FimArgs A) {
     __shared__ float tiles[kWaves][kTile8];  // (8+2)^3 at tix(x, y, z)
     __shared__ float hss[HYP ? kWaves : 1][512];  // h * slowness, tx + 8 ty + 64 z
     const int lane = threadIdx.x & 63;
-    float *tile = tiles[threadIdx.x >> 6];
-    float *hsl = hss[HYP ? (threadIdx.x >> 6) : 0];
-    const unsigned gw = blockIdx.x * kWaves + (threadIdx.x >> 6), G = gridDim.x * kWaves;
+    const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // this wave (scalar)
+    float *tile = tiles[wv];
+    float *hsl = hss[HYP ? wv : 0];
+    const unsigned gw = blockIdx.x * kWaves + wv, G = gridDim.x * kWaves;
     const int p = A.round & 1;
     unsigned incl = 0, count = 0;
     round_counts(A, lane, incl, count);
     if (gw == 0) {
         if (lane < kSeg) A.cnt[(((A.round + 2) % 3) * kSeg + lane) * kCntStride] = 0;
         if (lane == 0 && count) atomicAdd(&A.cnt[kRoundsIdx], 1u);
-        if (A.keys || A.tk)
-            for (int j = lane; j < A.nshot; j += 64) A.kmin[((A.round + 2) % 3) * A.nshot + j] = kInfBits;
+        if constexpr (KM)
+            for (int j = lane; j < A.ksub * A.kstride; j += 64)
+                A.kmin[((A.round + 2) % 3) * A.ksub * A.kstride + j] = kInfBits;
     }
     if (count == 0) return;
     const unsigned *cur = p ? A.list1 : A.list0;
@@ -532,7 +571,7 @@ __global__ __launch_bounds__(64 * kWaves, 6) void fim_round8(FimArgs A) {
     const int nbxy = A.nbx * A.nby;
     unsigned long long my_visits = 0, my_iters = 0, my_defer = 0;
 
-    for_items(A, count, incl, cur, nxt, nxt_cnt, bit_cur, bit_nxt, lane, gw, G, my_defer, [&](const unsigned item) {
+    for_items<KM>(A, count, incl, cur, nxt, nxt_cnt, bit_cur, bit_nxt, lane, gw, G, my_defer, [&](const unsigned item) {
         const unsigned shot = item >> kShotShift, b = item & kBlkMask;
         float *Tsh = A.T + (long long)shot * A.vol;
         unsigned *fl = A.flags + (long long)shot * A.nblk;
@@ -629,7 +668,7 @@ __global__ __launch_bounds__(64 * kWaves, 6) void fim_round8(FimArgs A) {
             const unsigned span = (unsigned)(zhi - zlo);
             const int i0 = tcol + kTZ * (kb + 1), h0 = lane + 64 * kb;
             // (indexed from the LDS arrays themselves: 32-bit addresses)
-            const int w = threadIdx.x >> 6;
+            const int w = wv;
 #pragma unroll
             for (int d = 0; d < 22; d++) {
                 if ((unsigned)(d - dlo) <= span) {
@@ -699,7 +738,8 @@ __global__ __launch_bounds__(64 * kWaves, 6) void fim_round8(FimArgs A) {
 
         // face activation as in the 4^3 kernel: a changed face cell must be
         // below the neighbour's adjacent cell (tile halo / z halo registers)
-        bool anydec = false, axl = false, ayl = false;
+        bool axl = false, ayl = false;
+        float most = 0.0f;   // largest decrease of the lane's cells
         // arrival-ordering keys: smallest activating value on the x faces
         // (tx = 0 / 7 lanes), the y faces (ty = 0 / 7) and among the changed
         // cells of the column
@@ -710,22 +750,30 @@ __global__ __launch_bounds__(64 * kWaves, 6) void fim_round8(FimArgs A) {
         #pragma unroll
         for (int k = 0; k < 8; k++) {
             const float dl = v0[k] - v[k];
-            anydec |= dl > 0.0f;
+            most = fmaxf(most, dl);
             const bool c = dl > A.eps;
             const int ti = tcol + kTZ * (k + 1);
-            const bool ax = c && xface && v[k] < tile[ti + ox];
-            const bool ay = c && yface && v[k] < tile[ti + oy];
-            axl |= ax;
-            ayl |= ay;
-            if (A.tk) {
-                kx = ax ? fminf(kx, v[k]) : kx;
-                ky = ay ? fminf(ky, v[k]) : ky;
-                kc = c ? fminf(kc, v[k]) : kc;
+            if constexpr (KM & 1) {
+                // through the values (an unchanged cell counts as +inf, which
+                // is below no halo): one short-lived mask at a time
+                const float t = c ? v[k] : kKeyInf;
+                kx = t < tile[ti + ox] ? fminf(kx, t) : kx;
+                ky = t < tile[ti + oy] ? fminf(ky, t) : ky;
+                kc = fminf(kc, t);
+            } else {
+                axl |= c && xface && v[k] < tile[ti + ox];
+                ayl |= c && yface && v[k] < tile[ti + oy];
             }
+        }
+        if constexpr (KM & 1) {
+            kx = xface ? kx : kKeyInf;
+            ky = yface ? ky : kKeyInf;
+            axl = kx < kKeyInf;
+            ayl = ky < kKeyInf;
         }
         const bool fzm = (v0[0] - v[0] > A.eps) && v[0] < vz[0];
         const bool fzp = (v0[7] - v[7] > A.eps) && v[7] < vz[9];
-        if (__ballot(anydec)) {
+        if (__ballot(most > 0.0f)) {
             #pragma unroll
             for (int k = 0; k < 8; k++) Tsh[base + lane + 64 * k] = v[k];
             if (A.xf) {
@@ -755,32 +803,40 @@ __global__ __launch_bounds__(64 * kWaves, 6) void fim_round8(FimArgs A) {
         default: break;
         }
         float key = kKeyInf;
-        if (A.tk) {
+        if constexpr (KM & 1) {
             // x faces: min over ty of the tx = 0 / 7 lanes (lanes tx + 8 ty;
             // row_ror 8 pairs ty with ty ^ 1 inside a row, readlane the rest);
             // y faces: min over tx of the ty = 0 / 7 rows of 8 lanes.  Only
             // for the faces that schedule a neighbour (the same in every lane)
-            float k0 = kKeyInf, k1 = kKeyInf, k2 = kKeyInf, k3 = kKeyInf, k4 = kKeyInf,
-                  k5 = kKeyInf, k6 = kKeyInf;
+            // (each selected into its lane at once: seven wave-uniform values
+            // kept side by side would not fit the scalar registers)
             if (xm || xp) {
                 const float mx = __uint_as_float(dpp_umin<0x128>(__float_as_uint(kx)));  // row_ror:8
-                k1 = fminf(fminf(lane_val(mx, 0), lane_val(mx, 16)),
-                           fminf(lane_val(mx, 32), lane_val(mx, 48)));
-                k2 = fminf(fminf(lane_val(mx, 7), lane_val(mx, 23)),
-                           fminf(lane_val(mx, 39), lane_val(mx, 55)));
+                const float k1 = fminf(fminf(lane_val(mx, 0), lane_val(mx, 16)),
+                                       fminf(lane_val(mx, 32), lane_val(mx, 48)));
+                const float k2 = fminf(fminf(lane_val(mx, 7), lane_val(mx, 23)),
+                                       fminf(lane_val(mx, 39), lane_val(mx, 55)));
+                key = lane == 1 ? k1 : lane == 2 ? k2 : key;
             }
             if (ym || yp) {
                 const float my = min8(ky);
-                k3 = lane_val(my, 0);
-                k4 = lane_val(my, 56);
+                const float k3 = lane_val(my, 0), k4 = lane_val(my, 56);
+                key = lane == 3 ? k3 : lane == 4 ? k4 : key;
             }
-            if (zm) k5 = wave_min_all(fzm ? v[0] : kKeyInf);
-            if (zp) k6 = wave_min_all(fzp ? v[7] : kKeyInf);
-            if (more) k0 = wave_min_all(kc);
-            key = lane == 0 ? k0 : lane == 1 ? k1 : lane == 2 ? k2 : lane == 3 ? k3
-                : lane == 4 ? k4 : lane == 5 ? k5 : k6;
+            if (zm) {
+                const float k5 = wave_min_all(fzm ? v[0] : kKeyInf);
+                key = lane == 5 ? k5 : key;
+            }
+            if (zp) {
+                const float k6 = wave_min_all(fzp ? v[7] : kKeyInf);
+                key = lane == 6 ? k6 : key;
+            }
+            if (more) {
+                const float k0 = wave_min_all(kc);
+                key = lane == 0 ? k0 : key;
+            }
         }
-        schedule(A, shot, fl, target, bit_nxt, nxt, nxt_cnt, lane, key);
+        schedule<KM>(A, shot, fl, target, bit_nxt, nxt, nxt_cnt, lane, gw, key);
         my_visits += 1;
         my_iters += it;
         wave_sync();
@@ -856,7 +912,7 @@ __global__ void seed_sources(const float *__restrict__ src, int nshot, const flo
                              float *T, unsigned *flags, unsigned *list0, unsigned *cnt,
                              float dx, float dy, float dz, int B, int nbx, int nby,
                              long long vol, long long nblk, const float *keys, unsigned *kmin,
-                             unsigned *tk, float *xf, int lazy) {
+                             int ksub, int kstride, unsigned *tk, float *xf, int lazy) {
     const int j = blockIdx.x * blockDim.x + threadIdx.x;
     if (j == 0) {  // the sources form segment 0 of the first list
         for (int k = 0; k < 3 * kSeg; k++) cnt[k * kCntStride] = 0;
@@ -887,15 +943,10 @@ __global__ void seed_sources(const float *__restrict__ src, int nshot, const flo
     }
     flags[(long long)j * nblk + b] = lazy ? 1u | 4u | (1u << 3) : 1u;
     list0[j] = ((unsigned)j << kShotShift) | b;
-    if (tk) {  // the source block opens the first list with key 0
-        tk[(long long)j * nblk + b] = 0u;
-        kmin[j] = keys ? __float_as_uint(keys[(long long)j * nblk + b]) : 0u;
-        kmin[nshot + j] = kInfBits;
-        kmin[2 * nshot + j] = kInfBits;
-    } else if (keys) {
-        kmin[j] = __float_as_uint(keys[(long long)j * nblk + b]);
-        kmin[nshot + j] = kInfBits;
-        kmin[2 * nshot + j] = kInfBits;
+    if (tk) tk[(long long)j * nblk + b] = 0u;  // the source block opens the first list with key 0
+    if (tk || keys) {
+        const unsigned first = keys ? __float_as_uint(keys[(long long)j * nblk + b]) : 0u;
+        for (int k = 0; k < 3 * ksub; k++) kmin[k * kstride + j] = k ? kInfBits : first;
     }
 }
 
@@ -1285,6 +1336,16 @@ __global__ __launch_bounds__(1024) void sum_wave_stats(const unsigned long long 
 // ---------------------------------------------------------------------------
 namespace st {
 
+// Words per shot's smallest key: eight lines of 32 shots' words between them.
+// With one line (up to 32 shots) a round's atomics queue for it: 16 shots of
+// 201 x 201 x 101 in arrival order take 6.9 ms with one word per shot and 3.4
+// with eight; from 256 shots on, one word is as fast to update and faster to
+// read (17.9 ms against 18.9 for 256 shots).
+static int key_words(int nshot) {
+    int k = kKeySub;
+    while (k > 1 && (nshot + 31) / 32 * k > 8) k /= 2;
+    return k;
+}
 static int blk_index(int B) { return B == 8 ? 1 : 0; }
 
 // The model's slowness in the block layout of edge B, into S (vol floats).
@@ -1331,7 +1392,8 @@ void fim_batch(st_ctx *ctx, const float *dsrc, int nshot, const st_fim_opts &o,
     const BlockGeo g = make_geo(ctx->nx, ctx->ny, ctx->nz, o.block);
     ctx->list[0].reserve(fim_list_bytes(g.nblk, nshot));
     ctx->list[1].reserve(fim_list_bytes(g.nblk, nshot));
-    if (keys || tentative) ctx->kmin.reserve(sizeof(unsigned) * 3 * std::max(nshot, 1));
+    const int ks = (nshot + 31) / 32 * 32;   // whole lines
+    if (keys || tentative) ctx->kmin.reserve(sizeof(unsigned) * 3 * kKeySub * std::max(ks, 32));
     if (tentative) ctx->tkeys.reserve(sizeof(unsigned) * 2 * nshot * g.nblk);
     if (stats) ctx->wstats.reserve(sizeof(unsigned long long) * 3 * fim_waves(o));
     if (o.block == 8) ctx->xfaces.reserve(sizeof(float) * 128 * g.nblk * nshot);
@@ -1342,6 +1404,8 @@ void fim_batch(st_ctx *ctx, const float *dsrc, int nshot, const st_fim_opts &o,
     bf.list0 = ctx->list[0].as<unsigned>();
     bf.list1 = ctx->list[1].as<unsigned>();
     bf.kmin = ctx->kmin.as<unsigned>();
+    bf.ksub = key_words(nshot);
+    bf.kstride = ks;
     bf.tk = ctx->tkeys.as<unsigned>();
     bf.wstats = ctx->wstats.as<unsigned long long>();
     bf.xf = o.block == 8 ? ctx->xfaces.as<float>() : nullptr;
@@ -1384,7 +1448,8 @@ void fim_batch_on(st_ctx *ctx, const FimBufs &bf, const float *dsrc, int nshot,
     ST_HIP(hipMemsetAsync(bf.flags, 0, sizeof(unsigned) * g.nblk * nshot, ctx->stream));
     hipLaunchKernelGGL(seed_sources, dim3((nshot + 63) / 64), dim3(64), 0, ctx->stream, dsrc,
                        nshot, bf.S, bf.T, bf.flags, bf.list0, cnt, ctx->dx, ctx->dy, ctx->dz, B,
-                       g.nbx, g.nby, g.vol, g.nblk, keys, bf.kmin, tk, xf, lazy ? 1 : 0);
+                       g.nbx, g.nby, g.vol, g.nblk, keys, bf.kmin, bf.ksub, bf.kstride, tk, xf,
+                       lazy ? 1 : 0);
     ST_HIP(hipGetLastError());
 
     FimArgs A;
@@ -1404,6 +1469,8 @@ void fim_batch_on(st_ctx *ctx, const FimBufs &bf, const float *dsrc, int nshot,
     A.max_inner = o.max_inner;
     A.keys = keys;
     A.kmin = bf.kmin;
+    A.ksub = bf.ksub;
+    A.kstride = bf.kstride;
     A.nshot = nshot;
     A.band = o.band;
     A.src = dsrc;
@@ -1434,13 +1501,15 @@ void fim_batch_on(st_ctx *ctx, const FimBufs &bf, const float *dsrc, int nshot,
     };
     const long long max_rounds = 4LL * (g.nbx + g.nby + g.nbz) * 64 + 4096;
     const bool hyp = o.sweep != 1;
+    // the round kernel of the block edge, the pass and the keys in use
+    void (*const round_kernels[3][4])(FimArgs) = {
+        {fim_round4<0>, fim_round4<1>, fim_round4<2>, fim_round4<3>},
+        {fim_round8<false, 0>, fim_round8<false, 1>, fim_round8<false, 2>, fim_round8<false, 3>},
+        {fim_round8<true, 0>, fim_round8<true, 1>, fim_round8<true, 2>, fim_round8<true, 3>}};
+    const auto round_kernel =
+        round_kernels[B == 8 ? (hyp ? 2 : 1) : 0][(A.tk ? 1 : 0) | (A.keys ? 2 : 0)];
     auto launch_round = [&](const FimArgs &a) {
-        if (B == 8 && hyp)
-            hipLaunchKernelGGL(fim_round8<true>, dim3(grid), dim3(64 * kWaves), 0, ctx->stream, a);
-        else if (B == 8)
-            hipLaunchKernelGGL(fim_round8<false>, dim3(grid), dim3(64 * kWaves), 0, ctx->stream, a);
-        else
-            hipLaunchKernelGGL(fim_round4, dim3(grid), dim3(64 * kWaves), 0, ctx->stream, a);
+        hipLaunchKernelGGL(round_kernel, dim3(grid), dim3(64 * kWaves), 0, ctx->stream, a);
     };
 
     ST_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
@@ -1456,7 +1525,7 @@ void fim_batch_on(st_ctx *ctx, const FimBufs &bf, const float *dsrc, int nshot,
         auto mix = [&](long long v) { key = (key ^ v) * 1099511628211LL; };
         mix((long long)(uintptr_t)A.T); mix((long long)(uintptr_t)A.S); mix((long long)(uintptr_t)A.keys);
         mix((long long)(uintptr_t)A.flags); mix((long long)(uintptr_t)A.list0);
-        mix((long long)(uintptr_t)A.list1); mix((long long)(uintptr_t)A.kmin);
+        mix((long long)(uintptr_t)A.list1); mix((long long)(uintptr_t)A.kmin); mix(A.ksub); mix(A.kstride);
         mix((long long)(uintptr_t)A.stats);
         mix(nshot); mix(B); mix(grid); mix(A.nblk); mix(A.max_inner);
         // every geometry field the kernels read: two models with the same

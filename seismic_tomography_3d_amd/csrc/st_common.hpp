@@ -163,13 +163,14 @@ void ensure_range(st_ctx *ctx);
 namespace st {
 // Device buffers of one batched FIM solve (sizes as fim_batch reserves them
 // for nshot shots: T nshot*vol, flags nshot*nblk, each list
-// fim_list_bytes(nblk, nshot), kmin 3*nshot, tk 2*nshot*nblk, wstats
+// fim_list_bytes(nblk, nshot), kmin 3*ksub*kstride, tk 2*nshot*nblk, wstats
 // 3*fim_waves(opts) counters).
 struct FimBufs {
     const float *S = nullptr;      // block-layout slowness
     float *T = nullptr;
     unsigned *flags = nullptr, *list0 = nullptr, *list1 = nullptr;
     unsigned *kmin = nullptr, *tk = nullptr;
+    int ksub = 1, kstride = 0;     // words per shot's smallest key and their stride (>= nshot)
     unsigned long long *wstats = nullptr;
     float *xf = nullptr;           // 8^3 blocks: copies of each block's two x faces
                                    // (nshot * nblk * 128 floats; nullable)
