@@ -12,10 +12,7 @@ namespace nn {
 
 // ---------------------------------------------------------------------------
 // GEMM  C[M,N] = A[M,K] * B[K,N]  (BF16 operands, FP32 accumulate)
-//   ta = 0: A(m,k) = A[m*lda + k]     ta = 1: A(m,k) = A[k*lda + m]
-//   tb = 0: B(k,n) = B[k*ldb + n]     tb = 1: B(k,n) = B[n*ldb + k]
-//   mode 0: C = act(acc + bias) (and a BF16 copy when C16 is set)
-//   mode 1: C += acc with atomics (split-K over blockIdx.z)
+//   A(m,k) = A[m*lda + k], B(k,n) = B[k*ldb + n]
 // 256 threads = 4 waves; 64x64 tile per workgroup, 32x32 per wave as 2x2
 // v_mfma_f32_16x16x16_bf16 tiles; K staged through LDS in steps of 32.
 // ---------------------------------------------------------------------------
@@ -29,32 +26,19 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const long long m0 = (long long)blockIdx.y * 64;
     const int n0 = blockIdx.x * 64;
-    const int kchunk = (((g.K + g.ksplit - 1) / g.ksplit) + 31) / 32 * 32;
-    const int kbeg = blockIdx.z * kchunk;
-    const int kend = min(g.K, kbeg + kchunk);
     f4v acc[2][2];
     for (int i = 0; i < 2; i++)
         for (int j = 0; j < 2; j++) acc[i][j] = f4v{0.f, 0.f, 0.f, 0.f};
     const int wm = (w >> 1) * 32, wn = (w & 1) * 32;
-    for (int k0 = kbeg; k0 < kend; k0 += 32) {
+    for (int k0 = 0; k0 < g.K; k0 += 32) {
         for (int e = tid; e < 2048; e += 256) {
-            int mm, kk;
-            if (!g.ta) { mm = e >> 5; kk = e & 31; } else { kk = e >> 6; mm = e & 63; }
+            const int mm = e >> 5, kk = e & 31, k = k0 + kk;
             const long long m = m0 + mm;
-            const int k = k0 + kk;
-            unsigned short v = 0;
-            if (m < g.M && k < kend)
-                v = g.ta ? g.A[(long long)k * g.lda + m] : g.A[m * g.lda + k];
-            As[mm][kk] = v;
+            As[mm][kk] = m < g.M && k < g.K ? g.A[m * g.lda + k] : (unsigned short)0;
         }
         for (int e = tid; e < 2048; e += 256) {
-            int nn, kk;
-            if (!g.tb) { kk = e >> 6; nn = e & 63; } else { nn = e >> 5; kk = e & 31; }
-            const int n = n0 + nn, k = k0 + kk;
-            unsigned short v = 0;
-            if (n < g.N && k < kend)
-                v = g.tb ? g.B[(long long)n * g.ldb + k] : g.B[(long long)k * g.ldb + n];
-            Bs[nn][kk] = v;
+            const int kk = e >> 6, nn = e & 63, n = n0 + nn, k = k0 + kk;
+            Bs[nn][kk] = n < g.N && k < g.K ? g.B[(long long)k * g.ldb + n] : (unsigned short)0;
         }
         __syncthreads();
         for (int ks = 0; ks < 32; ks += 16) {
@@ -82,20 +66,12 @@ __global__ __launch_bounds__(256) void gemm_bf16(GemmArgs g) {
                 const long long m = m0 + wm + i * 16 + 4 * (lane >> 4) + r;
                 const int n = n0 + wn + j * 16 + (lane & 15);
                 if (m >= g.M || n >= g.N) continue;
-                float v = acc[i][j][r];
-                if (g.mode == 1) {
-                    atomicAdd(&g.C[m * g.ldc + n], v);
-                } else {
-                    if (g.bias) v += g.bias[n];
-                    if (g.relu) v = fmaxf(v, 0.f);
-                    if (g.C) g.C[m * g.ldc + n] = v;
-                    if (g.C16) g.C16[m * g.ldc + n] = f2bf(v);
-                }
+                g.C[m * g.ldc + n] = acc[i][j][r];
             }
 }
 
 void gemm(hipStream_t st, const GemmArgs &g) {
-    dim3 grid((g.N + 63) / 64, (unsigned)((g.M + 63) / 64), g.ksplit);
+    dim3 grid((g.N + 63) / 64, (unsigned)((g.M + 63) / 64));
     hipLaunchKernelGGL(gemm_bf16, grid, dim3(256), 0, st, g);
     ST_HIP(hipGetLastError());
 }
@@ -386,6 +362,258 @@ __global__ __launch_bounds__(256) void conv3d_fwd(const void *__restrict__ X0v, 
     }
 }
 
+// ---------------------------------------------------------------------------
+// Convolution backward without an im2col matrix (its 27-fold copy of the
+// activations, written and read for each product, was most of the time: a
+// batch of 8 on the 32^3 cube took 10.2 ms).  Both kernels take bricks of 8 x 4
+// x 4 voxels and stage them in LDS; dY is the masked gradient in BF16, as the
+// products round it.
+// ---------------------------------------------------------------------------
+
+// Input gradient: dX[v, c] = sum_tap (sum_n dY[v - off(tap), n] W[tap, c, n]).
+// A workgroup holds the brick's dY halo, all channels n (padded to NP), and
+// computes CT tiles of 16 channels c: wave w the 16-voxel tiles w and w + 4.
+// Each tap's product runs through the 16-wide matrix instruction from zero and
+// is then added in tap order, the sums a product matrix summed over taps
+// gives, bit for bit: later layers' gradients round these to BF16.
+template <int KS, int NP, int CT>
+__global__ __launch_bounds__(256) void conv3d_bwd_x(const unsigned short *__restrict__ D,
+                                                    const unsigned short *__restrict__ Wb,
+                                                    float *__restrict__ dX, int e, int cin,
+                                                    int cout) {
+    constexpr int HF = KS / 2, HX = 8 + KS - 1, HY = 4 + KS - 1, NH = HX * HY * HY;
+    constexpr int NST = NP + 4, KC = NP / 16, TAPS = KS * KS * KS;
+    __shared__ __align__(16) unsigned short halo[NH * NST];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int nbx = (e + 7) / 8, nb4 = (e + 3) / 4;
+    int bid = blockIdx.x;
+    const int bx = bid % nbx; bid /= nbx;
+    const int by = bid % nb4; bid /= nb4;
+    const int bz = bid % nb4;
+    const long long V = (long long)e * e * e, base = (bid / nb4) * V;
+    const int ctt = gridDim.y * CT, ct0 = blockIdx.y * CT;
+    for (int i = tid; i < NH * (NP / 4); i += 256) {
+        const int hv = i / (NP / 4), n = (i - hv * (NP / 4)) * 4;
+        const int hx = hv % HX, hr = hv / HX;
+        const int x = 8 * bx + hx - HF, y = 4 * by + hr % HY - HF, z = 4 * bz + hr / HY - HF;
+        uint2 v = make_uint2(0u, 0u);
+        if (x >= 0 && y >= 0 && z >= 0 && x < e && y < e && z < e && n < cout) {
+            const unsigned short *p = D + (base + x + (long long)e * (y + (long long)e * z)) * cout + n;
+            if ((cout & 3) == 0) v = *reinterpret_cast<const uint2 *>(p);
+            else {
+                unsigned short h[4] = {0, 0, 0, 0};
+                for (int k = 0; k < 4 && n + k < cout; k++) h[k] = p[k];
+                v = make_uint2((unsigned)h[0] | ((unsigned)h[1] << 16),
+                               (unsigned)h[2] | ((unsigned)h[3] << 16));
+            }
+        }
+        *reinterpret_cast<uint2 *>(&halo[hv * NST + n]) = v;
+    }
+    __syncthreads();
+    const int m = lane & 15, q = lane >> 4;
+    // this lane's voxel of tile t: x = m & 7, y = 2 (t & 1) + (m >> 3), z = t >> 1
+    int hb[2];
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int mt = w + 4 * t;
+        hb[t] = ((m & 7) + HX * ((2 * (mt & 1) + (m >> 3)) + HY * (mt >> 1))) * NST + 4 * q;
+    }
+    f4v sum[2][CT];
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int j = 0; j < CT; j++) sum[t][j] = f4v{0.f, 0.f, 0.f, 0.f};
+    s4v b[2][KC][CT];
+    auto load_b = [&](int tap, s4v (&f)[KC][CT]) {
+#pragma unroll
+        for (int k = 0; k < KC; k++)
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+                f[k][j] = *reinterpret_cast<const s4v *>(
+                    Wb + (((long long)tap * KC + k) * ctt + ct0 + j) * 256 + lane * 4);
+    };
+    auto step = [&](int tap, const s4v (&f)[KC][CT]) {
+        const int tx = tap % KS, ty = (tap / KS) % KS, tz = tap / (KS * KS);
+        const int off = ((KS - 1 - tx) + HX * ((KS - 1 - ty) + HY * (KS - 1 - tz))) * NST;
+        f4v p[2][CT];
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int j = 0; j < CT; j++) p[t][j] = f4v{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int k = 0; k < KC; k++)
+#pragma unroll
+            for (int t = 0; t < 2; t++) {
+                const s4v a = *reinterpret_cast<const s4v *>(&halo[hb[t] + off + 16 * k]);
+#pragma unroll
+                for (int j = 0; j < CT; j++)
+                    p[t][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, f[k][j], p[t][j], 0, 0, 0);
+            }
+#pragma unroll
+        for (int t = 0; t < 2; t++)
+#pragma unroll
+            for (int j = 0; j < CT; j++) sum[t][j] += p[t][j];
+    };
+    // the next tap's weights travel with this tap's products.  (The tap index is
+    // opaque: fully unrolled, the loads of all taps are hoisted and spill.)
+    load_b(0, b[0]);
+    for (int tap = 0; tap < TAPS; tap += 2) {
+        asm volatile("" : "+s"(tap));
+        if (tap + 1 < TAPS) load_b(tap + 1, b[1]);
+        step(tap, b[0]);
+        if (tap + 1 >= TAPS) break;
+        if (tap + 2 < TAPS) load_b(tap + 2, b[0]);
+        step(tap + 1, b[1]);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; t++) {
+        const int mt = w + 4 * t;
+#pragma unroll
+        for (int j = 0; j < CT; j++) {
+            const int c = 16 * (ct0 + j) + m;
+            if (c >= cin) continue;
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int mo = 4 * q + r;
+                const int x = 8 * bx + (mo & 7), y = 4 * by + 2 * (mt & 1) + (mo >> 3),
+                          z = 4 * bz + (mt >> 1);
+                if (x < e && y < e && z < e)
+                    dX[(base + x + (long long)e * (y + (long long)e * z)) * cin + c] = sum[t][j][r];
+            }
+        }
+    }
+}
+
+// Wb of conv3d_bwd_x in fragment order: (tap, k group of 16, c tile) is 64
+// lanes x 4 BF16, lane = m + 16 q holding W[tap, c = 16 ct + m, n = 16 k + 4 q
+// + i]; zero past cin and cout.  W16 is [tap*cin + c][cout].
+__global__ void pack_conv_bwd(const unsigned short *__restrict__ W16,
+                              unsigned short *__restrict__ Wb, int taps, int cin, int cout, int kc,
+                              int ctt) {
+    const int tot = taps * kc * ctt * 256;
+    for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
+        const int u = i & 3, lane = (i >> 2) & 63, f = i >> 8;
+        const int ct = f % ctt, k = (f / ctt) % kc, tap = f / (ctt * kc);
+        const int c = 16 * ct + (lane & 15), n = 16 * k + 4 * (lane >> 4) + u;
+        Wb[i] = c < cin && n < cout ? W16[((long long)tap * cin + c) * cout + n] : (unsigned short)0;
+    }
+}
+
+// Weight gradient: dW[tap, c, n] += sum_w X[w, c] dY[w - off(tap), n], the
+// matrix instruction's k running over voxels.  A workgroup takes CT tiles of
+// 16 channels c and 16 channels n over every gridDim.x-th brick, wave w the
+// taps w, w + 4, ...: their accumulators stay in registers over all bricks and
+// are added to dW once.  X is staged [c][voxel], dY [n][row][x] with its halo
+// rows in three copies shifted by -1, 0, 1 along x, so every fragment (eight
+// voxels of a row) is one aligned 16-byte read; row strides of 136 and 328
+// halves put the 16 lanes of a fragment on distinct bank groups.
+template <int KS, int CT>
+__global__ __launch_bounds__(256) void conv3d_bwd_w(const float *__restrict__ X,
+                                                    const unsigned short *__restrict__ D,
+                                                    float *__restrict__ dW, int e, int cin,
+                                                    int cout, int nbrick, int cchunks) {
+    constexpr int HF = KS / 2, HX = 8 + KS - 1, HY = 4 + KS - 1, NROW = HY * HY;
+    constexpr int XST = 136, DST = (NROW * 8 + 16 + 31) / 32 * 32 + 8, TAPS = KS * KS * KS;
+    constexpr int TW = (TAPS + 3) / 4;
+    static_assert(KS != 3 || DST >= NROW * 8, "row stride");
+    __shared__ __align__(16) unsigned short sX[16 * CT * XST];
+    __shared__ __align__(16) unsigned short sD[KS][16 * DST];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int c0 = (blockIdx.y % cchunks) * 16 * CT, n0 = (blockIdx.y / cchunks) * 16;
+    const int nbx = (e + 7) / 8, nb4 = (e + 3) / 4;
+    const int m = lane & 15, q = lane >> 4;
+    f4v acc[TW][CT];
+#pragma unroll
+    for (int i = 0; i < TW; i++)
+#pragma unroll
+        for (int j = 0; j < CT; j++) acc[i][j] = f4v{0.f, 0.f, 0.f, 0.f};
+    for (int brick = blockIdx.x; brick < nbrick; brick += gridDim.x) {
+        int bid = brick;
+        const int bx = bid % nbx; bid /= nbx;
+        const int by = bid % nb4; bid /= nb4;
+        const int bz = bid % nb4;
+        const long long base = (long long)(bid / nb4) * e * e * e;
+        // X: voxel v = x + 8 (y + 4 z), four channels an item
+        for (int i = tid; i < 128 * 4 * CT; i += 256) {
+            const int v = i / (4 * CT), c = (i - v * 4 * CT) * 4;
+            const int x = 8 * bx + (v & 7), y = 4 * by + ((v >> 3) & 3), z = 4 * bz + (v >> 5);
+            float f[4] = {0.f, 0.f, 0.f, 0.f};
+            if (x < e && y < e && z < e && c0 + c < cin) {
+                const float *p = X + (base + x + (long long)e * (y + (long long)e * z)) * cin + c0 + c;
+                if ((cin & 3) == 0) {
+                    const float4 t = *reinterpret_cast<const float4 *>(p);
+                    f[0] = t.x; f[1] = t.y; f[2] = t.z; f[3] = t.w;
+                } else {
+                    for (int k = 0; k < 4; k++)
+                        if (c0 + c + k < cin) f[k] = p[k];
+                }
+            }
+#pragma unroll
+            for (int k = 0; k < 4; k++) sX[(c + k) * XST + v] = f2bf(f[k]);
+        }
+        // dY: copy t holds at x the value of x + HF - t (halo column x + KS - 1 - t)
+        for (int i = tid; i < HX * NROW * 4; i += 256) {
+            const int hv = i >> 2, n = (i & 3) * 4;
+            const int hx = hv % HX, row = hv / HX;
+            const int x = 8 * bx + hx - HF, y = 4 * by + row % HY - HF, z = 4 * bz + row / HY - HF;
+            unsigned short h[4] = {0, 0, 0, 0};
+            if (x >= 0 && y >= 0 && z >= 0 && x < e && y < e && z < e) {
+                const unsigned short *p =
+                    D + (base + x + (long long)e * (y + (long long)e * z)) * cout + n0 + n;
+                if ((cout & 3) == 0) {
+                    const uint2 t = *reinterpret_cast<const uint2 *>(p);
+                    h[0] = (unsigned short)t.x; h[1] = (unsigned short)(t.x >> 16);
+                    h[2] = (unsigned short)t.y; h[3] = (unsigned short)(t.y >> 16);
+                } else {
+                    for (int k = 0; k < 4; k++)
+                        if (n0 + n + k < cout) h[k] = p[k];
+                }
+            }
+#pragma unroll
+            for (int t = 0; t < KS; t++) {
+                const int xo = hx + t - (KS - 1);
+                if (xo >= 0 && xo < 8)
+#pragma unroll
+                    for (int k = 0; k < 4; k++) sD[t][(n + k) * DST + row * 8 + xo] = h[k];
+            }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {   // 32 voxels: z = ks, lane group q the row y = q
+            if (KS == 1 && ks != w) continue;
+            b8v a[CT];
+#pragma unroll
+            for (int j = 0; j < CT; j++)
+                a[j] = *reinterpret_cast<const b8v *>(&sX[(16 * j + m) * XST + 32 * ks + 8 * q]);
+#pragma unroll
+            for (int i = 0; i < TW; i++) {
+                const int tap = KS == 1 ? 0 : w + 4 * i;
+                if (tap >= TAPS) break;
+                const int tx = tap % KS, ty = (tap / KS) % KS, tz = tap / (KS * KS);
+                const int row = (ks + KS - 1 - tz) * HY + q + KS - 1 - ty;
+                const b8v b = *reinterpret_cast<const b8v *>(&sD[tx][m * DST + row * 8]);
+#pragma unroll
+                for (int j = 0; j < CT; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[j], b, acc[i][j], 0, 0, 0);
+            }
+        }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < TW; i++) {
+        const int tap = KS == 1 ? 0 : w + 4 * i;
+        if (tap >= TAPS) break;
+#pragma unroll
+        for (int j = 0; j < CT; j++)
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int c = c0 + 16 * j + 4 * q + r, n = n0 + m;
+                if (c < cin && n < cout)
+                    atomicAdd(&dW[((long long)tap * cin + c) * cout + n], acc[i][j][r]);
+            }
+    }
+}
+
 // Wp in MFMA fragment order: fragment (s, j) is 64 lanes x 8 BF16, lane =
 // m + 16 q holding W[k][n = 16 j + m] for k = 32 s + 8 q .. + 7, where
 // k = tap * cinp + c; zero where tap >= taps, n >= cout or c >= cin.  A
@@ -414,53 +642,6 @@ __global__ void pack_conv(const unsigned short *__restrict__ W16, unsigned short
 #define GRID_STRIDE(i, n) \
     for (long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x; i < (n); \
          i += (long long)gridDim.x * blockDim.x)
-
-// col[(s,v), tap*C + c] = X[s, v + off(tap), c] (zero outside), BF16
-__global__ void im2col3(const float *__restrict__ X, unsigned short *__restrict__ col, int ns,
-                        int n, int C, int ksz) {
-    const long long V = (long long)n * n * n;
-    const int taps = ksz * ksz * ksz, h = ksz / 2;
-    const long long total = (long long)ns * V * taps * C;
-    GRID_STRIDE(i, total) {
-        const int c = (int)(i % C);
-        long long r = i / C;
-        const int tap = (int)(r % taps);
-        const long long sv = r / taps;
-        const long long s = sv / V;
-        const int v = (int)(sv - s * V);
-        const int x = v % n, y = (v / n) % n, z = v / (n * n);
-        const int tx = tap % ksz - h, ty = (tap / ksz) % ksz - h, tz = tap / (ksz * ksz) - h;
-        const int xx = x + tx, yy = y + ty, zz = z + tz;
-        float val = 0.f;
-        if (xx >= 0 && yy >= 0 && zz >= 0 && xx < n && yy < n && zz < n)
-            val = X[(s * V + xx + (long long)n * (yy + (long long)n * zz)) * C + c];
-        col[i] = f2bf(val);
-    }
-}
-
-// dX[s, v, c] = sum_tap dcol[(s, v - off(tap)), tap*C + c]
-__global__ void col2im3(const float *__restrict__ dcol, float *__restrict__ dX, int ns, int n,
-                        int C, int ksz) {
-    const long long V = (long long)n * n * n;
-    const int taps = ksz * ksz * ksz, h = ksz / 2;
-    const long long total = (long long)ns * V * C;
-    GRID_STRIDE(i, total) {
-        const int c = (int)(i % C);
-        const long long sv = i / C;
-        const long long s = sv / V;
-        const int v = (int)(sv - s * V);
-        const int x = v % n, y = (v / n) % n, z = v / (n * n);
-        float acc = 0.f;
-        for (int tap = 0; tap < taps; tap++) {
-            const int tx = tap % ksz - h, ty = (tap / ksz) % ksz - h, tz = tap / (ksz * ksz) - h;
-            const int xx = x - tx, yy = y - ty, zz = z - tz;
-            if (xx < 0 || yy < 0 || zz < 0 || xx >= n || yy >= n || zz >= n) continue;
-            const long long src = s * V + xx + (long long)n * (yy + (long long)n * zz);
-            acc += dcol[(src * taps + tap) * C + c];
-        }
-        dX[i] = acc;
-    }
-}
 
 // 2x average pooling: out n/2 cube
 __global__ void avgpool2(const float *__restrict__ X, float *__restrict__ Y, int ns, int n, int C) {
@@ -561,31 +742,29 @@ __global__ void chan_copy(const float *__restrict__ X, float *__restrict__ Y, lo
     }
 }
 
-// dY *= (Y > 0), and a BF16 copy
-__global__ void relu_bwd(float *__restrict__ dY, const float *__restrict__ Y,
-                         unsigned short *__restrict__ d16, long long n, int relu) {
+// d16 = BF16 of dY (Y > 0), db[c] += sum_r of the masked gradient.  A thread's
+// elements are a multiple of C apart (C divides 256), so they share a channel
+// and neighbouring threads read neighbouring elements.
+__global__ __launch_bounds__(256) void relu_bias_bwd(const float *__restrict__ dY,
+                                                     const float *__restrict__ Y,
+                                                     unsigned short *__restrict__ d16,
+                                                     float *__restrict__ db, long long n, int C,
+                                                     int relu) {
+    __shared__ float sh[256];
+    float acc = 0.f;
     GRID_STRIDE(i, n) {
         float d = dY[i];
         if (relu && !(Y[i] > 0.f)) d = 0.f;
-        dY[i] = d;
         d16[i] = f2bf(d);
+        acc += d;
     }
-}
-
-// db[c] += sum_r dY[r, c]
-__global__ void bias_grad(const float *__restrict__ dY, float *__restrict__ db, long long rows, int C) {
-    __shared__ float sh[256];
-    const int c = blockIdx.y;
-    float acc = 0.f;
-    for (long long r = (long long)blockIdx.x * 256 + threadIdx.x; r < rows; r += (long long)gridDim.x * 256)
-        acc += dY[r * C + c];
     sh[threadIdx.x] = acc;
     __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
+    for (int o = 128; o >= C; o >>= 1) {
         if (threadIdx.x < o) sh[threadIdx.x] += sh[threadIdx.x + o];
         __syncthreads();
     }
-    if (threadIdx.x == 0) atomicAdd(&db[c], sh[0]);
+    if (threadIdx.x < C) atomicAdd(&db[threadIdx.x], sh[threadIdx.x]);
 }
 
 // weighted MSE with under-predictions weighted wu: w = m (p < t ? wu : 1),
@@ -645,14 +824,6 @@ static unsigned blocks_for(long long n) {
 // ---------------------------------------------------------------------------
 // host wrappers
 // ---------------------------------------------------------------------------
-void im2col(hipStream_t st, const float *X, unsigned short *col, int ns, int n, int C, int ksz) {
-    const long long tot = (long long)ns * n * n * n * ksz * ksz * ksz * C;
-    hipLaunchKernelGGL(im2col3, dim3(blocks_for(tot)), dim3(256), 0, st, X, col, ns, n, C, ksz);
-}
-void col2im(hipStream_t st, const float *dcol, float *dX, int ns, int n, int C, int ksz) {
-    const long long tot = (long long)ns * n * n * n * C;
-    hipLaunchKernelGGL(col2im3, dim3(blocks_for(tot)), dim3(256), 0, st, dcol, dX, ns, n, C, ksz);
-}
 void pool(hipStream_t st, const float *X, float *Y, int ns, int n, int C) {
     hipLaunchKernelGGL(avgpool2, dim3(blocks_for((long long)ns * n * n * n / 8 * C)), dim3(256), 0,
                        st, X, Y, ns, n, C);
@@ -678,12 +849,12 @@ void chancopy(hipStream_t st, const float *X, float *Y, long long rows, int C, i
     hipLaunchKernelGGL(chan_copy, dim3(blocks_for(rows * C)), dim3(256), 0, st, X, Y, rows, C, Ctot,
                        off, backward ? 1 : 0);
 }
-void relu_backward(hipStream_t st, float *dY, const float *Y, unsigned short *d16, long long n,
-                   bool relu) {
-    hipLaunchKernelGGL(relu_bwd, dim3(blocks_for(n)), dim3(256), 0, st, dY, Y, d16, n, relu ? 1 : 0);
-}
-void bias_gradient(hipStream_t st, const float *dY, float *db, long long rows, int C) {
-    hipLaunchKernelGGL(bias_grad, dim3(64, C), dim3(256), 0, st, dY, db, rows, C);
+void relu_bias_backward(hipStream_t st, const float *dY, const float *Y, unsigned short *d16,
+                        float *db, long long rows, int C, bool relu) {
+    ST_REQUIRE(C >= 1 && 256 % C == 0, ST_ERR_ARG, "channels must divide 256");
+    const unsigned b = blocks_for(rows * C);
+    hipLaunchKernelGGL(relu_bias_bwd, dim3(b < 512 ? b : 512), dim3(256), 0, st, dY, Y, d16, db,
+                       rows * C, C, relu ? 1 : 0);
 }
 void mse_loss(hipStream_t st, const float *p, const float *t, const float *m, float *grad,
               double *acc, long long n, float under_weight) {
@@ -717,6 +888,74 @@ void pack_conv_weights(hipStream_t st, const unsigned short *W16, unsigned short
     hipLaunchKernelGGL(pack_conv, dim3(blocks_for(tot)), dim3(256), 0, st, W16, Wp, taps, cin,
                        cout, conv_cinp(cin), conv_coutp(cout));
     ST_HIP(hipGetLastError());
+}
+
+// tiles of 16 input channels one workgroup of the backward kernels takes
+static int bwd_tiles(int cin) {
+    const int t = (cin + 15) / 16;
+    return t <= 4 ? t : (t % 4 == 0 ? 4 : 3);
+}
+static int bwd_bricks(int ns, int e) {
+    const long long n = (long long)ns * ((e + 7) / 8) * ((e + 3) / 4) * ((e + 3) / 4);
+    ST_REQUIRE(n < (1LL << 31), ST_ERR_ARG, "conv grid too large");
+    return (int)n;
+}
+long long conv_bwd_packed_size(int ksz, int cin, int cout) {
+    return (long long)ksz * ksz * ksz * ((cout + 15) / 16) * ((cin + 15) / 16) * 256;
+}
+
+void conv_backward_input(hipStream_t st, const unsigned short *D, const unsigned short *W16,
+                         unsigned short *Wb, float *dX, int ns, int e, int cin, int cout, int ksz) {
+    const int kc = (cout + 15) / 16, ctt = (cin + 15) / 16, ct = bwd_tiles(cin);
+    const int taps = ksz * ksz * ksz, nb = bwd_bricks(ns, e);
+    ST_REQUIRE(ctt % ct == 0, ST_ERR_ARG, "conv channels");
+    if (nb == 0) return;
+    hipLaunchKernelGGL(pack_conv_bwd, dim3(blocks_for(conv_bwd_packed_size(ksz, cin, cout))),
+                       dim3(256), 0, st, W16, Wb, taps, cin, cout, kc, ctt);
+    const dim3 g(nb, ctt / ct), b(256);
+#define ST_BWD_X(KS, NP, CT)                                                                      \
+    if (ksz == KS && kc * 16 == NP && ct == CT) {                                                 \
+        hipLaunchKernelGGL((conv3d_bwd_x<KS, NP, CT>), g, b, 0, st, D, Wb, dX, e, cin, cout);     \
+        ST_HIP(hipGetLastError());                                                                \
+        return;                                                                                   \
+    }
+    ST_BWD_X(3, 16, 1)
+    ST_BWD_X(3, 32, 1)
+    ST_BWD_X(3, 32, 2)
+    ST_BWD_X(3, 64, 2)
+    ST_BWD_X(3, 64, 4)
+    ST_BWD_X(3, 32, 3)
+    ST_BWD_X(3, 16, 3)
+    ST_BWD_X(1, 16, 1)
+#undef ST_BWD_X
+    ST_REQUIRE(false, ST_ERR_ARG, "no convolution kernel for this channel configuration");
+}
+
+void conv_backward_weight(hipStream_t st, const float *X, const unsigned short *D, float *dW,
+                          int ns, int e, int cin, int cout, int ksz) {
+    const int nt = (cout + 15) / 16, ctt = (cin + 15) / 16, ct = bwd_tiles(cin);
+    const int nb = bwd_bricks(ns, e), cchunks = ctt / ct;
+    ST_REQUIRE(ctt % ct == 0, ST_ERR_ARG, "conv channels");
+    if (nb == 0) return;
+    // two workgroups per CU over all channel groups, each adding its sums once;
+    // fewer for the 1^3 head, whose few sums would queue (512: 113 us at 262,144
+    // voxels)
+    const int gx = std::max(1, std::min(nb, (ksz == 1 ? 64 : 512) / (cchunks * nt)));
+    const dim3 g(gx, cchunks * nt), b(256);
+#define ST_BWD_W(KS, CT)                                                                          \
+    if (ksz == KS && ct == CT) {                                                                  \
+        hipLaunchKernelGGL((conv3d_bwd_w<KS, CT>), g, b, 0, st, X, D, dW, e, cin, cout, nb,       \
+                           cchunks);                                                              \
+        ST_HIP(hipGetLastError());                                                                \
+        return;                                                                                   \
+    }
+    ST_BWD_W(3, 1)
+    ST_BWD_W(3, 2)
+    ST_BWD_W(3, 3)
+    ST_BWD_W(3, 4)
+    ST_BWD_W(1, 1)
+#undef ST_BWD_W
+    ST_REQUIRE(false, ST_ERR_ARG, "no convolution kernel for this channel configuration");
 }
 
 void conv_forward_any(hipStream_t st, const void *X0, int C0, bool up0, const void *X1, int C1,

@@ -23,17 +23,12 @@ struct GemmArgs {
     const unsigned short *A;
     const unsigned short *B;
     float *C;
-    unsigned short *C16;
-    const float *bias;
     long long M;
     int N, K;
     long long lda, ldb, ldc;
-    int ta, tb, relu, mode, ksplit;
 };
 
 void gemm(hipStream_t st, const GemmArgs &g);
-void im2col(hipStream_t st, const float *X, unsigned short *col, int ns, int n, int C, int ksz);
-void col2im(hipStream_t st, const float *dcol, float *dX, int ns, int n, int C, int ksz);
 void pool(hipStream_t st, const float *X, float *Y, int ns, int n, int C);
 void pool_bf16(hipStream_t st, const unsigned short *X, unsigned short *Y, int ns, int n, int C);
 void pool_bwd(hipStream_t st, const float *dY, float *dX, int ns, int n, int C);
@@ -41,9 +36,8 @@ void upsample(hipStream_t st, const float *X, float *Y, int ns, int m, int C, in
 void upsample_bwd(hipStream_t st, const float *dY, float *dX, int ns, int m, int C, int Ctot, int off);
 void chancopy(hipStream_t st, const float *X, float *Y, long long rows, int C, int Ctot, int off,
               bool backward);
-void relu_backward(hipStream_t st, float *dY, const float *Y, unsigned short *d16, long long n,
-                   bool relu);
-void bias_gradient(hipStream_t st, const float *dY, float *db, long long rows, int C);
+void relu_bias_backward(hipStream_t st, const float *dY, const float *Y, unsigned short *d16,
+                        float *db, long long rows, int C, bool relu);
 void mse_loss(hipStream_t st, const float *p, const float *t, const float *m, float *grad,
               double *acc, long long n, float under_weight);
 void adam_step(hipStream_t st, float *w, const float *g, float *m, float *v, unsigned short *w16,
@@ -58,7 +52,15 @@ void pack_conv_weights(hipStream_t st, const unsigned short *W16, unsigned short
                        int cin, int cout);
 void conv_forward(hipStream_t st, const float *X, const unsigned short *Wp, const float *bias,
                   float *Y, int ns, int e, int cin, int cout, int ksz, bool relu);
-// the same with the input the concatenation [X0 (C0 channels, nearest-
+// gradients of the same convolution from D, the masked output gradient in
+// BF16: dX written (Wb: conv_bwd_packed_size entries of scratch for the
+// re-ordered weights W16), dW [tap*cin + c][cout] added to
+long long conv_bwd_packed_size(int ksz, int cin, int cout);
+void conv_backward_input(hipStream_t st, const unsigned short *D, const unsigned short *W16,
+                         unsigned short *Wb, float *dX, int ns, int e, int cin, int cout, int ksz);
+void conv_backward_weight(hipStream_t st, const float *X, const unsigned short *D, float *dW,
+                          int ns, int e, int cin, int cout, int ksz);
+// the forward pass with the input the concatenation [X0 (C0 channels, nearest-
 // upsampled from half resolution when up0) | X1 (C1 channels)]
 void conv_forward2(hipStream_t st, const float *X0, int C0, bool up0, const float *X1, int C1,
                    const unsigned short *Wp, const float *bias, float *Y, int ns, int e, int cout,

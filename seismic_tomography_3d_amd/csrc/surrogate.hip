@@ -74,7 +74,7 @@ struct Net {
     DevBuf in0, a1, a2, p1, a3, a4, p2, a5, p3, a7, cat3, a8, cat2, a9, cat1, a10, out;
     DevBuf d_out, d_a10, d_cat1, d_a9, d_a2, d_t32, d_cat2, d_a8, d_a4, d_t16, d_cat3, d_a7, d_a5,
         d_t8, d_p3, d_p2, d_a3, d_p1, d_a1, d_in;
-    DevBuf col, dcol, d16, lossacc;
+    DevBuf d16, wb, lossacc;
     // training set
     DevBuf X, Y, M, bX, bY, bM, Q;
     long long nsamples = 0;
@@ -98,7 +98,7 @@ void surrogate_release(st_ctx *ctx) {
                       &n.p2, &n.a5, &n.p3, &n.a7, &n.cat3, &n.a8, &n.cat2, &n.a9, &n.cat1, &n.a10,
                       &n.out, &n.d_out, &n.d_a10, &n.d_cat1, &n.d_a9, &n.d_a2, &n.d_t32, &n.d_cat2,
                       &n.d_a8, &n.d_a4, &n.d_t16, &n.d_cat3, &n.d_a7, &n.d_a5, &n.d_t8, &n.d_p3,
-                      &n.d_p2, &n.d_a3, &n.d_p1, &n.d_a1, &n.d_in, &n.col, &n.dcol, &n.d16,
+                      &n.d_p2, &n.d_a3, &n.d_p1, &n.d_a1, &n.d_in, &n.d16, &n.wb,
                       &n.lossacc, &n.X, &n.Y, &n.M, &n.bX, &n.bY, &n.bM, &n.Q})
         b->release();
     delete &s;
@@ -151,8 +151,8 @@ static void net_alloc_params(st_ctx *ctx, Net &n, unsigned seed) {
 
 __host__ __device__ inline long long cube(int e) { return (long long)e * e * e; }
 
-// forward buffers for ns samples; with train also the gradient and im2col
-// buffers of the backward pass
+// forward buffers for ns samples; with train also the buffers of the backward
+// pass
 static void net_alloc_batch(Net &n, int ns, bool train) {
     const int e1 = n.nc, e2 = n.nc / 2, e4 = n.nc / 4, e8 = n.nc / 8;
     const long long v1 = cube(e1) * ns, v2 = cube(e2) * ns, v4 = cube(e4) * ns, v8 = cube(e8) * ns;
@@ -170,15 +170,13 @@ static void net_alloc_batch(Net &n, int ns, bool train) {
     F(n.d_a4, v2 * 32); F(n.d_t16, v2 * 32); F(n.d_cat3, v4 * 128); F(n.d_a7, v8 * 64);
     F(n.d_a5, v4 * 64); F(n.d_t8, v4 * 64); F(n.d_p3, v8 * 64); F(n.d_p2, v4 * 32);
     F(n.d_a3, v2 * 32); F(n.d_p1, v2 * 16); F(n.d_a1, v1 * 16); F(n.d_in, v1 * kIn);
-    long long colmax = 0, ymax = 0;
+    long long ymax = 0, wmax = 0;
     for (auto &c : n.L) {
-        const long long V = cube(n.nc / c.res_div) * ns;
-        colmax = std::max(colmax, V * c.ksz * c.ksz * c.ksz * c.cin);
-        ymax = std::max(ymax, V * c.cout);
+        ymax = std::max(ymax, cube(n.nc / c.res_div) * ns * c.cout);
+        wmax = std::max(wmax, nn::conv_bwd_packed_size(c.ksz, c.cin, c.cout));
     }
-    n.col.reserve(sizeof(unsigned short) * colmax);
-    n.dcol.reserve(sizeof(float) * colmax);
     n.d16.reserve(sizeof(unsigned short) * ymax);
+    n.wb.reserve(sizeof(unsigned short) * wmax);
     n.lossacc.reserve(64);
     n.tcap = ns;
 }
@@ -210,38 +208,19 @@ static void net_pack(st_ctx *ctx, Net &n) {
     n.pver = n.wver;
 }
 
-// one convolution backward: dY (in place masked) -> dW, db (+=), dX (written)
-static void conv_bwd(st_ctx *ctx, Net &n, int li, const float *X, const float *Y, float *dY,
+// one convolution backward: dY -> dW, db (+=), dX (written)
+static void conv_bwd(st_ctx *ctx, Net &n, int li, const float *X, const float *Y, const float *dY,
                      float *dX, int ns) {
     const Conv &c = n.L[li];
     const int e = n.nc / c.res_div;
-    const int taps = c.ksz * c.ksz * c.ksz;
     const long long rows = cube(e) * ns;
     unsigned short *d16 = n.d16.as<unsigned short>();
-    nn::relu_backward(ctx->stream, dY, Y, d16, rows * c.cout, c.relu);
-    nn::bias_gradient(ctx->stream, dY, n.g.as<float>() + c.ob, rows, c.cout);
-    nn::im2col(ctx->stream, X, n.col.as<unsigned short>(), ns, e, c.cin, c.ksz);
-    // dW[taps*cin, cout] += col^T dY
-    nn::GemmArgs gw{};
-    gw.A = n.col.as<unsigned short>();
-    gw.ta = 1; gw.lda = (long long)taps * c.cin;
-    gw.B = d16; gw.tb = 0; gw.ldb = c.cout;
-    gw.C = n.g.as<float>() + c.ow; gw.ldc = c.cout;
-    gw.M = (long long)taps * c.cin; gw.N = c.cout; gw.K = (int)rows;
-    gw.mode = 1;
-    gw.ksplit = (int)std::min<long long>(512, std::max<long long>(1, rows / 2048));
-    nn::gemm(ctx->stream, gw);
-    if (dX) {
-        // dcol[rows, taps*cin] = dY W^T
-        nn::GemmArgs gd{};
-        gd.A = d16; gd.ta = 0; gd.lda = c.cout;
-        gd.B = n.w16.as<unsigned short>() + c.ow; gd.tb = 1; gd.ldb = c.cout;
-        gd.C = n.dcol.as<float>(); gd.ldc = (long long)taps * c.cin;
-        gd.M = rows; gd.N = taps * c.cin; gd.K = c.cout;
-        gd.ksplit = 1;
-        nn::gemm(ctx->stream, gd);
-        nn::col2im(ctx->stream, n.dcol.as<float>(), dX, ns, e, c.cin, c.ksz);
-    }
+    nn::relu_bias_backward(ctx->stream, dY, Y, d16, n.g.as<float>() + c.ob, rows, c.cout, c.relu);
+    nn::conv_backward_weight(ctx->stream, X, d16, n.g.as<float>() + c.ow, ns, e, c.cin, c.cout,
+                             c.ksz);
+    if (dX)
+        nn::conv_backward_input(ctx->stream, d16, n.w16.as<unsigned short>() + c.ow,
+                                n.wb.as<unsigned short>(), dX, ns, e, c.cin, c.cout, c.ksz);
 }
 
 __global__ void add_into(float *__restrict__ y, const float *__restrict__ x, long long n) {
@@ -924,7 +903,7 @@ int st_nn_gemm(st_ctx *ctx, const float *A, const float *B, float *C, int M, int
         g.A = a16.as<unsigned short>(); g.lda = K;
         g.B = b16.as<unsigned short>(); g.ldb = N;
         g.C = c.as<float>(); g.ldc = N;
-        g.M = M; g.N = N; g.K = K; g.ksplit = 1;
+        g.M = M; g.N = N; g.K = K;
         nn::gemm(ctx->stream, g);
         ST_HIP(hipMemcpyAsync(C, c.ptr, sizeof(float) * M * N, hipMemcpyDeviceToHost, ctx->stream));
         ST_HIP(hipStreamSynchronize(ctx->stream));
