@@ -29,11 +29,14 @@
 // rounded up to nzp, a multiple of 32, so that rows start on 128-byte lines
 // and every tile row segment is whole lines; the cells z >= nzz of a row are
 // padding (zero, never read).
-// V^2 dt^2 and the damper are two such volumes shared by all shots; per
-// shot three rotating wavefields.  A cell's damper is formed from the 1D
+// V^2 dt^2 is one such volume shared by all shots; per shot two wavefields:
+// a cell's U_pas is read only by the thread that then writes its U_fut, so
+// U_fut takes its place.  A cell's damper is formed from the 1D
 // profile (nb floats) in the reference's accumulation order, not stored.  A
 // step reads U_pre, U_pas and V^2 dt^2 once per cell and writes U_fut once:
 // 16 bytes per cell and step.
+#include <algorithm>
+#include <climits>
 #include <cmath>
 #include <cstring>
 #include <type_traits>
@@ -96,15 +99,28 @@ __device__ __forceinline__ float damper_of(float vz, bool iz, float vx, bool ix,
     return n == 0 ? 1.0f : (n == 1 ? d1v : (n == 2 ? d2 : d3));
 }
 
+// The correctly rounded a / b for every float a, with y the smallest double
+// that is not below 1 / b: q = a y lies at the exact quotient or at most two
+// units of its last place beyond it, and clearing two bits leaves an error
+// below 2^-50 of it.  A quotient of two floats is nearer than 2^-49 to a
+// value halfway between floats only if it is that value; it is one only
+// below the normal range, has its low bits zero there, and is what the
+// clearing returns.  So the conversion rounds as the division does, with
+// zeros, infinities and NaN along the way: four instructions where the
+// division takes eleven, one of them at a quarter of the rate.
+__device__ __forceinline__ float div_exact(float a, double y) {
+    const double q = (double)a * y;
+    return (float)__longlong_as_double(__double_as_longlong(q) & ~3LL);
+}
+
 // -------------------------------------------------------------------------
 // the time step
 
 struct StepArgs {
     const float *cv;       // V^2 dt^2, padded volume
     const float *d1;       // 1D damping profile (nb)
-    const float *prev;     // undamped U_pre of step t-1, shot stride N
-    const float *cur;      // U_pre of step t (without the wavelet)
-    float *out;            // U_fut of step t
+    const float *cur;      // U_pre of step t (without the wavelet), shot stride N
+    float *out;            // undamped U_pre of step t-1, replaced by U_fut of step t
     const long long *sid;  // source cell per shot
     long long N;           // cells per padded volume
     int nzz, nzp, nzr, nxx, nyy;   // nzr: nzz rounded up to 4 (the last quad)
@@ -112,34 +128,39 @@ struct StepArgs {
     int ntz, ntx;          // tiles along z and x
     int nchunks, ychunk;   // chunks of y planes and their length
     float wcur, wprev;     // wavelet[t], wavelet[t-1] (0 at t = 0)
-    float den_x, den_y, den_z;   // 5040 d^2
+    double inv_x, inv_y, inv_z;   // 1 / (5040 d^2), rounded up (div_exact)
+    // receivers of step t-1, read from cur by the workgroups behind the tiles
+    const long long *rcell;
+    float *rec;            // rec[t-1][g][r]
+    int nrec, rblocks;     // receivers, workgroups per shot (0: none)
+    unsigned tblocks;      // workgroups that step tiles
 };
 
 typedef float f4 __attribute__((ext_vector_type(4)));
 
-// Buffer resource over the cells [first, N) of one volume (raw buffer,
-// 32-bit byte offsets; a load past the end returns 0 instead of faulting)
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t vol_rsrc(const float *base, long long first,
-                                                           long long N) {
-    const long long bytes = (N - first) * 4;
-    const unsigned num = bytes > 0xffffffffLL ? 0xffffffffu : (unsigned)bytes;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(base + first), (short)0, (int)num,
-                                             0x00020000);
+// quads at a byte offset from a uniform base
+__device__ __forceinline__ f4 ld4(const float *base, unsigned off) {
+    return *reinterpret_cast<const f4 *>(reinterpret_cast<const char *>(base) + off);
 }
-__device__ __forceinline__ f4 bld4(__amdgpu_buffer_rsrc_t r, unsigned off) {
-    return __builtin_bit_cast(f4, __builtin_amdgcn_raw_buffer_load_b128(r, (int)off, 0, 0));
-}
-__device__ __forceinline__ void bst1(__amdgpu_buffer_rsrc_t r, unsigned off, float v) {
-    __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(unsigned, v), r, (int)off, 0, 0);
-}
-__device__ __forceinline__ void bst4(__amdgpu_buffer_rsrc_t r, unsigned off, f4 v) {
-    __builtin_amdgcn_raw_buffer_store_b128(
-        __builtin_bit_cast(__attribute__((ext_vector_type(4))) unsigned, v), r, (int)off, 0, 0);
+__device__ __forceinline__ void st4(float *base, unsigned off, f4 v) {
+    *reinterpret_cast<f4 *>(reinterpret_cast<char *>(base) + off) = v;
 }
 
 template <class F, int... J>
 __device__ __forceinline__ void unrolled(F &&f, std::integer_sequence<int, J...>) {
     (f(std::integral_constant<int, J>{}), ...);
+}
+
+// buildSeismogram (acoustic.cpp:325-334): a step's sample of every receiver
+// of G shots, rec[g][r]
+__device__ __forceinline__ void record_cells(const float *__restrict__ out, long long N,
+                                             const long long *__restrict__ rcell, int nrec, int r,
+                                             int g, float *rec) {
+    if (r < nrec) rec[(long long)g * nrec + r] = out[g * N + rcell[r]];
+}
+__global__ void wave_record(const float *__restrict__ out, long long N,
+                            const long long *__restrict__ rcell, int nrec, float *rec) {
+    record_cells(out, N, rcell, nrec, blockIdx.x * blockDim.x + threadIdx.x, blockIdx.y, rec);
 }
 
 // One workgroup advances a tile of 4 LZ (z) x TX (x) cells of one shot
@@ -155,6 +176,13 @@ __device__ __forceinline__ void unrolled(F &&f, std::integer_sequence<int, J...>
 // take two 16-byte LDS reads, its x-neighbours eight.  Workgroups are
 // numbered so that each XCD (workgroup id mod 8) receives a contiguous run
 // of tiles: x-neighbours, which share halo rows, run on the same L2.
+// The workgroups behind the tiles record the previous step's field, which
+// this step only reads: 5 us a step as a launch of its own, nothing here.
+// Vector issue bounds the step (about 300 instructions a wave and plane, two
+// thirds of its time), then the memory floor of 30 us for the 16 bytes a
+// cell.  One shot of 241 x 221 x 181 padded cells: 69 us a step before, with
+// IEEE divisions (427 instructions), a damper's axis flags in spilled
+// scalars, rebuilt buffer descriptors and 32-plane chunks; 37 us now.
 template <int LZ>
 __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
     constexpr int RW = 64 / LZ;            // x rows per wave
@@ -165,8 +193,14 @@ __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
     __shared__ f4 tb[2][HX][HZ4];
     __shared__ f4 td[2][HX][HZ4];
 
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const int total = gridDim.x, pblk = blockIdx.x, full = total & ~7;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if (blockIdx.x >= a.tblocks) {
+        const int rb = blockIdx.x - a.tblocks, g = rb / a.rblocks;
+        record_cells(a.cur, a.N, a.rcell, a.nrec, (rb - g * a.rblocks) * 256 + tid, g, a.rec);
+        return;
+    }
+    const int total = a.tblocks, pblk = blockIdx.x, full = total & ~7;
     const int logical = pblk < full ? (pblk & 7) * (full >> 3) + (pblk >> 3) : pblk;
     const int ntiles = a.ntz * a.ntx, per_shot = ntiles * a.nchunks;
     const int shot = logical / per_shot, rem = logical - shot * per_shot;
@@ -177,7 +211,7 @@ __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
     const int nzp = a.nzp;
     const long long NXZ = (long long)nzp * a.nxx, N = a.N;
     const long long so = (long long)shot * N;
-    const float *cur = a.cur + so, *prev = a.prev + so;
+    const float *cur = a.cur + so;
     float *out = a.out + so;
     // the source: plane ks, byte offset cs in the plane, cell sj of its quad
     const long long sq = a.sid[shot];
@@ -194,68 +228,69 @@ __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
     const unsigned col = (unsigned)(min(z, a.nzr - 4) + min(x, a.nxx - 1) * nzp) * 4u;
     // quads are aligned and the interior starts at z = 4: a quad is either
     // below it or starts inside it (and may end past it)
-    bool comp[4];
-#pragma unroll
-    for (int j = 0; j < 4; j++) comp[j] = z >= 4 && z + j < a.nzz - 4 && x < a.nxx - 4;
-    const bool any = comp[0];
-    const bool all4 = comp[3];
+    const int ncomp = z >= 4 && x < a.nxx - 4 ? min(max(a.nzz - 4 - z, 0), 4) : 0;
+    const bool any = ncomp > 0;
+    const bool all4 = ncomp == 4;
     // halo quads: x halo (4 rows before the tile, damped; 4 after) by waves
     // 0 and 1 (LZ = 16) or wave 0 (LZ = 8); z halo (one quad below each row,
-    // damped; one above) by wave 2
-    const bool xh_on = tid < NXH;
-    const int xhr = tid / LZ, xhz = tid % LZ;          // halo row 0..7
-    const bool xleft = xhr < 4;
-    const int xhx = xleft ? x0 - 4 + xhr : min(x0 + TX + xhr - 4, a.nxx - 1);
-    const unsigned oxh = (unsigned)(min(z0 + 4 * xhz, a.nzr - 4) + xhx * nzp) * 4u;
-    const int xlrow = xleft ? xhr : TX + xhr;
-    const bool zh_on = w == 2 && lane < 2 * TX;
-    const bool zbelow = lane < TX;
-    const int zhrow = zbelow ? lane : lane - TX;
-    const int zhz = zbelow ? max(z0 - 4, 0) : min(z0 + TZ, a.nzr - 4);
-    const unsigned ozh = (unsigned)(zhz + min(x0 + min(zhrow, TX - 1), a.nxx - 1) * nzp) * 4u;
-    const int zhcol = zbelow ? 0 : LZ + 1;
+    // damped; one above) by wave 2.  A lane has at most one.
+    const bool xh_on = tid < NXH, h_on = xh_on || (w == 2 && lane < 2 * TX);
+    const bool hlow = xh_on ? tid / LZ < 4 : lane < TX;   // before / below: damped
+    int hx, hz;                            // its first cell
+    f4 *hdst[2];                           // its place in the two LDS planes
+    if (xh_on) {
+        const int hr = tid / LZ;           // halo row 0..7
+        hx = hlow ? x0 - 4 + hr : min(x0 + TX + hr - 4, a.nxx - 1);
+        hz = min(z0 + 4 * (tid % LZ), a.nzr - 4);
+        const int r = hlow ? hr : TX + hr;
+        for (int b = 0; b < 2; b++) hdst[b] = hlow ? &td[b][r][tid % LZ + 1] : &tb[b][r][tid % LZ + 1];
+    } else {
+        const int hr = hlow ? lane : lane - TX;
+        hx = min(x0 + min(hr, TX - 1), a.nxx - 1);
+        hz = hlow ? max(z0 - 4, 0) : min(z0 + TZ, a.nzr - 4);
+        const int r = min(hr, TX - 1) + 4;
+        for (int b = 0; b < 2; b++) hdst[b] = hlow ? &td[b][r][0] : &tb[b][r][LZ + 1];
+    }
+    const unsigned oh = (unsigned)(hz + hx * nzp) * 4u;
 
-    // profile values of the fixed axes: own row and quad, the x-halo row
-    // and quad, the z-halo quad below
+    // Dampers of a quad: its profile values along z and x, and its dampers in
+    // the planes y outside the absorbing layer, which do not depend on y
     const int nb = a.nb;
     auto lidx = [&](int i, int n) { return i < nb ? i : (i >= n - nb ? n - 1 - i : -1); };
-    auto prof = [&](int l) { return l >= 0 ? a.d1[l] : 0.0f; };
-    const int lxo = lidx(min(x, a.nxx - 1), a.nxx);
-    const float vxo = prof(lxo);
-    float vzo[4], vzh[4], vzb[4];
-    int lzo[4], lzh[4], lzb[4];
+    auto prof = [&](int l) { return l >= 0 ? a.d1[l] : -1.0f; };   // -1: not in the layer
+    struct Quad {
+        float vz[4], vx;
+        f4 in;
+    };
+    auto quad_of = [&](int zf, int xf) {
+        Quad q;
+        q.vx = prof(lidx(xf, a.nxx));
 #pragma unroll
-    for (int j = 0; j < 4; j++) {
-        lzo[j] = lidx(min(z, a.nzr - 4) + j, a.nzz);
-        vzo[j] = prof(lzo[j]);
-        lzh[j] = lidx(min(z0 + 4 * xhz, a.nzr - 4) + j, a.nzz);
-        vzh[j] = prof(lzh[j]);
-        lzb[j] = lidx(max(z0 - 4, 0) + j, a.nzz);
-        vzb[j] = prof(lzb[j]);
-    }
-    const int lxh = lidx(xhx, a.nxx), lxb = lidx(min(x0 + min(zhrow, TX - 1), a.nxx - 1), a.nxx);
-    const float vxh = prof(lxh), vxb = prof(lxb);
-    // dampers of a quad in plane k
-    auto quad_damper = [&](const float *vz, const int *lz, float vx, int lx, int k) {
-        const int ly = lidx(k, a.nyy);
-        const float vy = prof(ly);
+        for (int j = 0; j < 4; j++) {
+            q.vz[j] = prof(lidx(zf + j, a.nzz));
+            q.in[j] = damper_of(q.vz[j], q.vz[j] != -1.0f, q.vx, q.vx != -1.0f, 0.0f, false);
+        }
+        return q;
+    };
+    const Quad own = quad_of(min(z, a.nzr - 4), min(x, a.nxx - 1)), halo = quad_of(hz, hx);
+    // in plane k: ly its depth in the layer (uniform), vy its profile value
+    auto quad_damper = [&](const Quad &q, int ly, float vy) {
+        if (ly < 0) return q.in;
         f4 d;
 #pragma unroll
-        for (int j = 0; j < 4; j++) d[j] = damper_of(vz[j], lz[j] >= 0, vx, lx >= 0, vy, ly >= 0);
+        for (int j = 0; j < 4; j++) d[j] = damper_of(q.vz[j], q.vz[j] != -1.0f, q.vx, q.vx != -1.0f, vy, true);
         return d;
     };
 
     struct Pf {
-        f4 c, p, xh, zh;
+        f4 c, p, h;
     };
     Pf pf[2];
     auto fetch = [&](Pf &f, int k) {
         const long long first = (long long)k * NXZ;
-        const auto Rb = vol_rsrc(cur, first, N);
-        f.c = bld4(vol_rsrc(a.cv, first, N), col);
-        f.p = bld4(vol_rsrc(prev, first, N), col);
-        if (xh_on) f.xh = bld4(Rb, oxh);
-        if (zh_on) f.zh = bld4(Rb, ozh);
+        f.c = ld4(a.cv + first, col);
+        f.p = ld4(out + first, col);
+        if (h_on) f.h = ld4(cur + first, oh);
     };
     // add the wavelet to the source cell of a quad of U_pre of plane k
     auto inject = [&](f4 v, int k, unsigned off, float wv) {
@@ -267,9 +302,9 @@ __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
 #pragma unroll
     for (int m = 0; m < 9; m++) {
         const int k = kb - 4 + m;
-        const long long first = (long long)k * NXZ;
-        f4 v = inject(bld4(vol_rsrc(cur, first, N), col), k, col, a.wcur);
-        q[m] = m < 4 ? v * quad_damper(vzo, lzo, vxo, lxo, k) : v;
+        const f4 v = inject(ld4(cur + (long long)k * NXZ, col), k, col, a.wcur);
+        const int ly = lidx(k, a.nyy);
+        q[m] = m < 4 ? v * quad_damper(own, ly, prof(ly)) : v;
     }
     fetch(pf[0], kb);
 
@@ -281,28 +316,22 @@ __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
             if (k >= ke) return;
             Pf &cu = pf[b];
             if (k == ks) {   // uniform: the source plane
-                if (xh_on) cu.xh = inject(cu.xh, k, oxh, a.wcur);
-                if (zh_on) cu.zh = inject(cu.zh, k, ozh, a.wcur);
+                if (h_on) cu.h = inject(cu.h, k, oh, a.wcur);
                 cu.p = inject(cu.p, k, col, a.wprev);
             }
             const f4 u = q[C];
-            const f4 dk = quad_damper(vzo, lzo, vxo, lxo, k);
+            const int ly = lidx(k, a.nyy);
+            const float vy = prof(ly);
+            const f4 dk = quad_damper(own, ly, vy);
             const f4 ud = u * dk;
             tb[b][row + 4][zq + 1] = u;
             td[b][row + 4][zq + 1] = ud;
-            if (xh_on) {
-                if (xleft) td[b][xlrow][xhz + 1] = cu.xh * quad_damper(vzh, lzh, vxh, lxh, k);
-                else tb[b][xlrow][xhz + 1] = cu.xh;
-            }
-            if (zh_on) {
-                if (zbelow) td[b][zhrow + 4][zhcol] = cu.zh * quad_damper(vzb, lzb, vxb, lxb, k);
-                else tb[b][zhrow + 4][zhcol] = cu.zh;
-            }
+            if (h_on) *hdst[b] = hlow ? cu.h * quad_damper(halo, ly, vy) : cu.h;
             __syncthreads();
             const bool more = k + 1 < ke;
             if (more) {
                 fetch(pf[b ^ 1], k + 1);
-                q[NEW] = bld4(vol_rsrc(cur, (long long)(k + 5) * NXZ, N), col);
+                q[NEW] = ld4(cur + (long long)(k + 5) * NXZ, col);
             }
             if (any) {
                 const f4 zlo = td[b][row + 4][zq], zhi = tb[b][row + 4][zq + 2];
@@ -339,19 +368,20 @@ __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
                     sz = sz - 1008.0f * (zn[4 + jj - 2] + zp[4 + jj + 2]);
                     sz = sz + 8064.0f * (zn[4 + jj - 1] + zp[4 + jj + 1]);
                     sz = sz - 14350.0f * uc;
-                    const float lap = (sx / a.den_x + sy / a.den_y) + sz / a.den_z;
+                    const float lap = (div_exact(sx, a.inv_x) + div_exact(sy, a.inv_y)) +
+                                      div_exact(sz, a.inv_z);
                     const float pas = cu.p[jj] * dk[jj];
                     float f = cu.c[jj] * lap + 2.0f * uc;
                     f = f - pas;
                     res[jj] = f * dk[jj];
                 }
-                const auto Ro = vol_rsrc(out, (long long)k * NXZ, N);
+                float *const o = out + (long long)k * NXZ;
                 if (all4) {
-                    bst4(Ro, col, res);
+                    st4(o, col, res);
                 } else {
 #pragma unroll
-                    for (int jj = 0; jj < 4; jj++)
-                        if (comp[jj]) bst1(Ro, col + 4u * jj, res[jj]);
+                    for (int jj = 0; jj < 3; jj++)
+                        if (jj < ncomp) o[col / 4 + jj] = res[jj];
                 }
             }
             // the centre moves behind (damped); the loaded plane gets its wavelet
@@ -359,16 +389,6 @@ __global__ __launch_bounds__(256) void wave_step(StepArgs a) {
             if (more && k + 5 == ks) q[NEW] = inject(q[NEW], k + 5, col, a.wcur);
         }, std::make_integer_sequence<int, 10>{});
     }
-}
-
-// buildSeismogram (acoustic.cpp:325-334): sample t of every receiver of G
-// shots, stored time-major rec[t][g][r]
-__global__ void wave_record(const float *__restrict__ out, long long N,
-                            const long long *__restrict__ rcell, int nrec, int G, float *rec,
-                            int t) {
-    const int r = blockIdx.x * blockDim.x + threadIdx.x, g = blockIdx.y;
-    if (r >= nrec) return;
-    rec[((long long)t * G + g) * nrec + r] = out[g * N + rcell[r]];
 }
 
 // rec[t][g][r] -> seis[g][r][t] (the reference's seismogram[t + r nt])
@@ -592,10 +612,17 @@ std::vector<long long> cells(const WaveState &w, const float *p, int n, const ch
     return c;
 }
 
-template <int LZ> void launch_step(hipStream_t st, const StepArgs &a, int shots) {
-    const long long n = (long long)shots * a.ntz * a.ntx * a.nchunks;
-    ST_REQUIRE(n < (1LL << 31), ST_ERR_ARG, "acoustic model too large for one launch");
-    hipLaunchKernelGGL((wave_step<LZ>), dim3((unsigned)n), dim3(256), 0, st, a);
+// the smallest double not below 1 / b (div_exact)
+double inverse_up(float b) {
+    const double y = 1.0 / (double)b;
+    return std::fma(y, (double)b, -1.0) < 0 ? std::nextafter(y, HUGE_VAL) : y;
+}
+
+template <int LZ> void launch_step(hipStream_t st, StepArgs &a, int shots) {
+    const long long n = (long long)shots * a.ntz * a.ntx * a.nchunks, m = n + (long long)shots * a.rblocks;
+    ST_REQUIRE(m < (1LL << 31), ST_ERR_ARG, "acoustic model too large for one launch");
+    a.tblocks = (unsigned)n;
+    hipLaunchKernelGGL((wave_step<LZ>), dim3((unsigned)m), dim3(256), 0, st, a);
 }
 
 }  // namespace
@@ -701,20 +728,37 @@ void wave_shots(st_ctx *ctx, const float *wavelet, int nt, const float *src_xyz,
     a.ntx = (nxi + TXT - 1) / TXT;
     const long long tiles = (long long)a.ntz * a.ntx;
     // shots per launch: enough workgroups (about 2048, 8 per CU) with chunks
-    // of at least 32 planes; three wavefields per shot, at most 24 GiB
+    // of at least 32 planes; two wavefields per shot, at most 24 GiB
     int G = group;
     if (G == 0) {
         const long long wg1 = tiles * std::max(1, nyi / 32);
         G = (int)std::max<long long>(1, (2048 + wg1 - 1) / wg1);
     }
     G = std::min(G, nshot);
-    G = (int)std::max<long long>(1, std::min<long long>(G, (24LL << 30) / (12 * N)));
-    const long long chunks = std::max<long long>(1, (2048 + G * tiles - 1) / (G * tiles));
-    a.ychunk = (int)std::min<long long>(nyi, std::max<long long>(32, (nyi + chunks - 1) / chunks));
+    G = (int)std::max<long long>(1, std::min<long long>(G, (24LL << 30) / (8 * N)));
+    // planes per workgroup: the chunk length whose busiest CU is done first.
+    // A chunk of y planes costs y + 4 plane times (the ring's first nine
+    // planes are read before the first step), a plane time shared by three
+    // resident workgroups is the unit, and two or one of them leave a tenth
+    // or a third of the CU idle.  One shot of 141 x 121 x 81 cells and 50
+    // layer cells (45 tiles, 213 planes): 32 planes (the former rule's
+    // minimum, 1.2 workgroups per CU) 48 ms for 801 steps, 20: 35, 16: 33,
+    // 13 (765 workgroups, chosen) 30, 10: 38, 8: 34.
+    int ncu = 0;
+    ST_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
+    long long best = LLONG_MAX;
+    for (int y = std::min(4, nyi); y <= nyi; y++) {
+        const long long per_cu = (G * tiles * ((nyi + y - 1) / y) + ncu - 1) / ncu;
+        const long long cost = per_cu * (y + 4) * (per_cu == 1 ? 15 : per_cu == 2 ? 11 : 10);
+        if (cost <= best) {
+            best = cost;
+            a.ychunk = y;
+        }
+    }
     a.nchunks = (nyi + a.ychunk - 1) / a.ychunk;
-    a.den_x = w.den[0]; a.den_y = w.den[1]; a.den_z = w.den[2];
+    a.inv_x = inverse_up(w.den[0]); a.inv_y = inverse_up(w.den[1]); a.inv_z = inverse_up(w.den[2]);
     const int ngroups = (nshot + G - 1) / G;
-    w.fields.reserve(sizeof(float) * 3 * G * N);
+    w.fields.reserve(sizeof(float) * 2 * G * N);
     w.rcell.reserve(sizeof(long long) * nrec);
     w.sid.reserve(sizeof(long long) * G);
     w.rec.reserve(sizeof(float) * (size_t)nt * G * nrec);
@@ -722,29 +766,31 @@ void wave_shots(st_ctx *ctx, const float *wavelet, int nt, const float *src_xyz,
     if (picks_out) w.picks.reserve(sizeof(float) * (size_t)G * nrec);
     ST_HIP(hipMemcpyAsync(w.rcell.ptr, rc.data(), sizeof(long long) * nrec,
                           hipMemcpyHostToDevice, ctx->stream));
-    float *F[3] = {w.fields.as<float>(), w.fields.as<float>() + G * N,
-                   w.fields.as<float>() + 2 * G * N};
+    float *F[2] = {w.fields.as<float>(), w.fields.as<float>() + G * N};
     a.sid = w.sid.as<long long>();
+    a.rcell = w.rcell.as<long long>();
+    a.nrec = nrec;
+    auto rec_at = [&](int t) { return w.rec.as<float>() + (long long)std::max(t, 0) * G * nrec; };
     ST_HIP(hipEventRecord(w.ev[0], ctx->stream));
     for (int gi = 0; gi < ngroups; gi++) {
         const int gs = std::min(G, nshot - gi * G);
         ST_HIP(hipMemcpyAsync(w.sid.ptr, sc.data() + (size_t)gi * G, sizeof(long long) * gs,
                               hipMemcpyHostToDevice, ctx->stream));
-        ST_HIP(hipMemsetAsync(w.fields.ptr, 0, sizeof(float) * 3 * G * N, ctx->stream));
-        int ip = 0, ic = 1, io = 2;   // U_pas source, U_pre, U_fut
+        ST_HIP(hipMemsetAsync(w.fields.ptr, 0, sizeof(float) * 2 * G * N, ctx->stream));
+        int ic = 0, io = 1;   // U_pre; U_pas source and U_fut
         for (int t = 0; t < nt; t++) {
-            a.prev = F[ip];
             a.cur = F[ic];
             a.out = F[io];
             a.wcur = wavelet[t];
             a.wprev = t > 0 ? wavelet[t - 1] : 0.0f;
+            a.rblocks = t > 0 ? (nrec + 255) / 256 : 0;
+            a.rec = rec_at(t - 1);
             if (LZ == 16) launch_step<16>(ctx->stream, a, gs);
             else launch_step<8>(ctx->stream, a, gs);
-            hipLaunchKernelGGL(wave_record, dim3((nrec + 255) / 256, gs), dim3(256), 0, ctx->stream,
-                               F[io], N, w.rcell.as<long long>(), nrec, G, w.rec.as<float>(), t);
-            const int tmp = ip;
-            ip = ic; ic = io; io = tmp;
+            std::swap(ic, io);
         }
+        hipLaunchKernelGGL(wave_record, dim3((nrec + 255) / 256, gs), dim3(256), 0, ctx->stream,
+                           F[ic], N, w.rcell.as<long long>(), nrec, rec_at(nt - 1));
         ST_HIP(hipGetLastError());
         hipLaunchKernelGGL(wave_transpose, dim3((nt + 31) / 32, (nrec + 31) / 32, gs), dim3(256), 0,
                            ctx->stream, w.rec.as<float>(), w.seis.as<float>(), nt, G, nrec);
