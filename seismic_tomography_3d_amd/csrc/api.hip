@@ -265,7 +265,7 @@ int st_ctx_destroy(st_ctx *ctx) {
     if (ctx->graph) (void)hipGraphDestroy(ctx->graph);
     for (auto *b : {&ctx->slow_zxy, &ctx->range, &ctx->slow_blk[0], &ctx->slow_blk[1], &ctx->T, &ctx->flags,
                     &ctx->list[0], &ctx->list[1], &ctx->counters, &ctx->wstats, &ctx->fsm_S,
-                    &ctx->fsm_sid, &ctx->pod_T, &ctx->pod_stamp, &ctx->pod_list,
+                    &ctx->fsm_sid, &ctx->fsm_lists, &ctx->pod_T, &ctx->pod_stamp, &ctx->pod_list,
                     &ctx->pod_counts, &ctx->pod_nit,
                     &ctx->src, &ctx->rcv,
                     &ctx->picks, &ctx->scratch, &ctx->keys, &ctx->kmin, &ctx->judge, &ctx->pred,

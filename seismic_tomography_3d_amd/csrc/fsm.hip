@@ -24,15 +24,26 @@
 // once per block, in rows along z), the values along z stay in registers.
 // Each shot's source-bounded sweeps cover that shot's own boxes only.
 //
-// What bounds it: a step of the walk is about 100 (operators ruled out) to 240
-// dependent vector instructions, 400 to 1,000 cycles of one wave, so a lone
-// shot pays (blocks along the longest diagonal) x (zc + 15) such steps per
-// sweep, and a batch the vector issue of the lanes a block's skew leaves busy
-// (zc of zc + 15 steps).  Measured: one shot of 121 x 97 x 61 cells 21.1 ->
-// 6.5 ms, 64 shots of 201 x 201 x 101 77.5 -> 39.2 ms, against a launch per
-// plane of cells with the shots of a batch in the lanes.  Blocks of 14 cells
-// of z: 8 / 14 / 22 / 30 take 45 / 39 / 40 / 43 ms for the 64 shots (the tiles'
-// LDS against the idle lanes) and 7.2 / 7.4 / 7.9 / 7.8 for the lone one.
+// The full sweeps change few blocks (14 % of 64 shots of 201 x 201 x 101 in a
+// gradient, 12 to 65 % a sweep of other cases): each begins with a test of all
+// cells at once (fsm_test) against the times as they stand, which marks the
+// blocks with a cell that would be lowered.  The first cell of a sweep's order
+// to change in a block either was marked or reads a changed cell of an upwind
+// block, so a launch walks the marked blocks and those behind a face that has
+// changed, and every other block keeps the values the sweep would give it.
+// The blocks to walk are lists per diagonal, so that the waves of a launch are
+// its first workgroups and spread evenly; without lists the working blocks
+// fall unevenly on the SIMDs (33 us for a launch of 870 of them, 22 with).
+//
+// What bounds it: a step of the walk is about 210 vector instructions of one
+// wave, some 1,000 cycles, so a launch takes 16 us for a lone shot (4 of them
+// the launch itself) and there are (blocks along the longest diagonal) of
+// them per sweep; a batch adds the vector issue of the busiest SIMD.
+// Measured: one shot of 121 x 97 x 61 cells 21.1 ms with a launch per plane of
+// cells, 6.5 with all blocks walked, 5.0 now; 64 shots of 201 x 201 x 101 77.5,
+// 39.2, 25.5 ms (walks 20, tests 5.6).  Blocks of 9 / 11 / 14 / 15 / 22 cells of
+// z: 26.7 / 25.9 / 25.5 / 25.5 / 26.9 ms for the 64 shots, 4.8 / 4.9 / 5.0 /
+// 5.0 / 5.4 for the lone one.
 //
 // Layout: one padded volume per shot, z fastest.
 //
@@ -164,8 +175,8 @@ __device__ float fsm_update_any(float T, const FsmIn &c, const FsmGeo &g) {
 
 // The same update, bit for bit, in the ranges fsm_fast checks: square roots
 // and quotients by the spacing constants in their short correctly rounded
-// forms, and operators that cannot change the result left out.  With lim the
-// least of the cell's time and the 1D operators:
+// forms, and with PRUNE operators that cannot change the result left out.
+// With lim the least of the cell's time and the 1D operators:
 // * t3D is at least the weighted mean of its arms (its root is not negative
 //   and rounding is monotone), a linear form of the seven upwind times; above
 //   lim by more than rounding (2^-17 of the times) it is ruled out;
@@ -175,12 +186,13 @@ __device__ float fsm_update_any(float T, const FsmIn &c, const FsmGeo &g) {
 //   with 1 % of that term and 2^-16 of lim for rounding, at or above lim it
 //   is ruled out -- unless the 3D operator is in play, whose condition reads
 //   the 2D times.
-// In most of the sixteen sweeps a cell's front does not come from the sweep's
-// octant, and the operators fall away for whole waves.
-//
-// Branches are wave-uniform (any lane needs the operator), the lanes that do
-// not are masked by selects: a walk's steps depend on each other, and masked
-// branches cost more latency there than the instructions they skip.
+// In the full sweeps a cell's front mostly does not come from the sweep's
+// octant, and in their test the operators fall away for whole waves: branches
+// are wave-uniform (any lane needs the operator), the lanes that do not are
+// masked by selects.  A walk's lanes are cells that change, where some lane
+// needs each operator at nearly every step: without the tests a lone shot's
+// launch takes 16 us instead of 19, 64 shots 25.5 ms instead of 27.5.
+template <bool PRUNE>
 __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool on,
                                                  const FsmGeo &g) {
     const float dx = g.dx, dy = g.dy, dz = g.dz;
@@ -188,20 +200,23 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
     const float t1D = pmin(tv + dz * c.sv, pmin(te + dx * c.se, tn + dy * c.sn));
     const float latest = pmax(tv, pmax(te, tn));
     const float lim = pmin(T, t1D);
-    float l3 = __builtin_fmaf(g.wv, tv, c.tnve);
-    l3 = __builtin_fmaf(g.we, te, l3);
-    l3 = __builtin_fmaf(g.wn, tn, l3);
-    l3 = __builtin_fmaf(g.wev, c.tev, l3);
-    l3 = __builtin_fmaf(g.wen, c.ten, l3);
-    l3 = __builtin_fmaf(g.wnv, c.tnv, l3);
-    const float big = pmax(pmax(latest, c.tnve), pmax(c.tev, pmax(c.ten, c.tnv)));
-    const bool try3 = on & (t1D > latest) & (l3 < __builtin_fmaf(big + lim, 7.6293945e-6f, lim));
-    const float far2 = lim * 1.0000153f;
-    const bool pxz = try3 | (on & (__builtin_fmaf(c.sve, g.dmin, c.tev) < far2));
-    const bool pyz = try3 | (on & (__builtin_fmaf(c.svn, g.dmin, c.tnv) < far2));
-    const bool pxy = try3 | (on & (__builtin_fmaf(c.sen, g.dmin, c.ten) < far2));
+    bool try3 = true, pxz = true, pyz = true, pxy = true;
+    if (PRUNE) {
+        float l3 = __builtin_fmaf(g.wv, tv, c.tnve);
+        l3 = __builtin_fmaf(g.we, te, l3);
+        l3 = __builtin_fmaf(g.wn, tn, l3);
+        l3 = __builtin_fmaf(g.wev, c.tev, l3);
+        l3 = __builtin_fmaf(g.wen, c.ten, l3);
+        l3 = __builtin_fmaf(g.wnv, c.tnv, l3);
+        const float big = pmax(pmax(latest, c.tnve), pmax(c.tev, pmax(c.ten, c.tnv)));
+        try3 = on & (t1D > latest) & (l3 < __builtin_fmaf(big + lim, 7.6293945e-6f, lim));
+        const float far2 = lim * 1.0000153f;
+        pxz = try3 | (on & (__builtin_fmaf(c.sve, g.dmin, c.tev) < far2));
+        pyz = try3 | (on & (__builtin_fmaf(c.svn, g.dmin, c.tnv) < far2));
+        pxy = try3 | (on & (__builtin_fmaf(c.sen, g.dmin, c.ten) < far2));
+    }
     float t2D = 1e6f;
-    if (__any(pxz)) {
+    if (!PRUNE || __any(pxz)) {
         const bool ok = pxz & (tv < te + dx * c.sve) & (te < tv + dz * c.sve);
         const float ta = c.tev + te - tv;
         const float tb = c.tev - te + tv;
@@ -209,7 +224,7 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
         const float t = div_rn((tb * g.dz2i + ta * g.dx2i) + sqrt_rn(q), g.zx, g.rzx);
         t2D = ok ? t : t2D;
     }
-    if (__any(pyz)) {
+    if (!PRUNE || __any(pyz)) {
         const bool ok = pyz & (tv < tn + dy * c.svn) & (tn < tv + dz * c.svn);
         const float ta = tv - tn + c.tnv;
         const float tb = tn - tv + c.tnv;
@@ -217,7 +232,7 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
         const float t = div_rn((ta * g.dz2i + tb * g.dy2i) + sqrt_rn(q), g.zy, g.rzy);
         t2D = ok & (t < t2D) ? t : t2D;
     }
-    if (__any(pxy)) {
+    if (!PRUNE || __any(pxy)) {
         const bool ok = pxy & (te < tn + dy * c.sen) & (tn < te + dx * c.sen);
         const float ta = te - tn + c.ten;
         const float tb = tn - te + c.ten;
@@ -227,7 +242,7 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
     }
     float res = smin(lim, t2D);
     const bool use3 = try3 & (smin(t1D, t2D) > latest);
-    if (__any(use3)) {
+    if (!PRUNE || __any(use3)) {
         float ta, tb, tc;
         fsm_arms(c, ta, tb, tc);
         const float t2 = 9.0f * c.s * c.s * g.dsum;
@@ -317,9 +332,8 @@ __global__ void fsm_seed(float *__restrict__ T, const float *__restrict__ S,
 
 // One diagonal D of one sweep's blocks, for all shots.  Blocks are (A, B, C)
 // = distances from the start corner of the shot's box in units of zc cells
-// along z and eight along x and y; workgroup q holds shot q % nshot of block
-// (a0 + r % na, D - A - C, c0 + r / na), r = q / nshot.  A shot whose box has
-// no such block leaves at once.
+// along z and eight along x and y; workgroup q walks entry q / 8 of the list
+// of residue q % 8, and leaves at once where the list is shorter.
 //
 // The LDS tiles hold planes 0 (the upwind halo) .. 8 along x and y and 0 ..
 // zc along z, in sweep order.  P even and Q = 9 mod 16 put the 64 lanes of a
@@ -336,24 +350,137 @@ template <int LZ> struct FsmTile {
     static constexpr int N = 9 * Q;
 };
 
-template <int LZ, bool FAST>
+// The blocks a sweep has to walk, in a list per diagonal D = A + B + C and per
+// residue of shot + B (workgroups of one residue run on one XCD).  A block is
+// its number ((shot nC + C) nB + B) nA + A.
+struct FsmQueue {
+    unsigned *list;         // [D][8][cap]
+    unsigned *count;        // [D][8] of this sweep
+    unsigned *flag;         // per block, the full sweep it was last marked in
+    unsigned cap;
+    int sweep;              // 1 .. 8
+    int nA, nB, nC;
+    __device__ unsigned number(int shot, int A, int B, int C) const {
+        return ((unsigned)(shot * nC + C) * nB + B) * nA + A;
+    }
+    __device__ void put(int shot, int A, int B, int C) const {
+        const int e = (A + B + C) * 8 + ((shot + B) & 7);
+        list[(long long)e * cap + atomicAdd(count + e, 1u)] = number(shot, A, B, C);
+    }
+    // the same for a block that several may list
+    __device__ void put_once(int shot, int A, int B, int C) const {
+        unsigned *f = flag + number(shot, A, B, C);
+        if (__builtin_nontemporal_load(f) != (unsigned)sweep &&
+            atomicExch(f, (unsigned)sweep) != (unsigned)sweep)
+            put(shot, A, B, C);
+    }
+};
+
+// The blocks a sweep starts with: all blocks of the shots' boxes if it is
+// source-bounded, the marked ones if not; one thread per block of the largest
+// box.
+__global__ __launch_bounds__(256) void fsm_list(const int *__restrict__ sid, int nshot, FsmGeo g,
+                                                FsmSweep w, int zc, FsmQueue q) {
+    const long long id = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int shot = (int)(id / ((long long)q.nA * q.nB * q.nC));
+    if (shot >= nshot || (!w.init && q.flag[id] != (unsigned)q.sweep)) return;
+    const int r = (int)(id - (long long)shot * q.nA * q.nB * q.nC);
+    const int A = r % q.nA, B = r / q.nA % q.nB, C = r / (q.nA * q.nB);
+    int s0, zl, xl, yl;
+    sweep_axis(w.tz, w.init, g.nzz, sid[3 * shot], s0, zl);
+    sweep_axis(w.tx, w.init, g.nxx, sid[3 * shot + 1], s0, xl);
+    sweep_axis(w.ty, w.init, g.nyy, sid[3 * shot + 2], s0, yl);
+    if (zc * A < zl && 8 * B < xl && 8 * C < yl) q.put(shot, A, B, C);
+}
+
+// Whether a cell of a full sweep would be lowered by the times as they stand,
+// for all cells at once: marks the blocks that hold one.  Lanes run over the
+// (z, x) cells of the box in memory order, each walks the eight y planes of a
+// block, the times and voxels of one plane serving as the next one's upwind
+// ones.  w.init = 0: all shots sweep the same box.
+template <bool FAST>
+__global__ __launch_bounds__(256) void fsm_test(const float *__restrict__ T,
+                                                const float *__restrict__ S, FsmGeo g, FsmSweep w,
+                                                int zc, FsmQueue queue) {
+    int zs, zl, xs, xl, ys, yl;
+    sweep_axis(w.tz, 0, g.nzz, 0, zs, zl);
+    sweep_axis(w.tx, 0, g.nxx, 0, xs, xl);
+    sweep_axis(w.ty, 0, g.nyy, 0, ys, yl);
+    const int q = blockIdx.x * blockDim.x + threadIdx.x;
+    const bool on = q < zl * xl;
+    const int b = on ? q / zl : 0, a = on ? q - b * zl : 0;
+    const int C = blockIdx.y, shot = blockIdx.z;
+    const int i = zs + w.tz * a, j = xs + w.tx * b;
+    const int bz = w.tz < 0, bx = w.tx < 0, by = w.ty < 0;
+    // a cell and its upwind neighbours, a voxel and its upwind neighbours
+    const int t00 = i + g.nzz * j, t10 = t00 - w.tz, t01 = t00 - w.tx * g.nzz, t11 = t01 - w.tz;
+    const int iu = i - w.tz - bz, id = max(i - bz, 0);
+    const int ju = j - w.tx - bx, jd = max(j - bx, 0);
+    const int s00 = id + g.nzz * jd, s10 = iu + g.nzz * jd, s01 = id + g.nzz * ju,
+              s11 = iu + g.nzz * ju;
+    const long long plane = (long long)g.nxx * g.nzz;
+    const float *Ts = T + shot * g.nB;
+    const int y1 = ys + w.ty * (8 * C), nc = min(8, yl - 8 * C);
+    const float *Tk = Ts + plane * (y1 - w.ty), *Sk = S + plane * (y1 - w.ty - by);
+    float u00 = Tk[t00], u10 = Tk[t10], u01 = Tk[t01], u11 = Tk[t11];
+    float v00 = Sk[s00], v10 = Sk[s10], v01 = Sk[s01], v11 = Sk[s11];
+    bool hit = false;
+    for (int c = 0; c < nc; c++) {
+        const int k = y1 + w.ty * c;
+        Tk = Ts + plane * k;
+        Sk = S + plane * max(k - by, 0);
+        const float n00 = Tk[t00], n10 = Tk[t10], n01 = Tk[t01], n11 = Tk[t11];
+        const float m00 = Sk[s00], m10 = Sk[s10], m01 = Sk[s01], m11 = Sk[s11];
+        FsmIn f;
+        f.tv = n10;
+        f.te = n01;
+        f.tev = n11;
+        f.tn = u00;
+        f.tnv = u10;
+        f.ten = u01;
+        f.tnve = u11;
+        f.sve = pmin(m11, v11);
+        f.svn = pmin(v11, v10);
+        f.sen = pmin(v11, v01);
+        f.sv = pmin(f.sve, pmin(m10, v10));
+        f.se = pmin(f.sve, pmin(m01, v01));
+        f.sn = pmin(f.svn, pmin(v01, v00));
+        f.s = v11;
+        const float res = FAST ? fsm_update_fast<true>(n00, f, on, g) : fsm_update_any(n00, f, g);
+        hit |= !(res == n00);
+        u00 = n00;
+        u10 = n10;
+        u01 = n01;
+        u11 = n11;
+        v00 = m00;
+        v10 = m10;
+        v01 = m01;
+        v11 = m11;
+    }
+    if (hit & on) queue.flag[queue.number(shot, a / zc, b / 8, C)] = queue.sweep;
+}
+
+template <int LZ, bool FAST, bool FULL>
 __global__ __launch_bounds__(64) void fsm_block(float *__restrict__ T,
                                                 const float *__restrict__ S,
-                                                const int *__restrict__ sid, int nshot, FsmGeo g,
-                                                FsmSweep w, int zc, int D, int a0, int na, int c0) {
+                                                const int *__restrict__ sid, FsmGeo g,
+                                                FsmSweep w, int zc, int D, FsmQueue queue) {
     using Tile = FsmTile<LZ>;
     constexpr int P = Tile::P, Q = Tile::Q;
     __shared__ float tt[Tile::N + 1];
     __shared__ float ts[Tile::N];
-    const int shot = blockIdx.x % nshot, r = blockIdx.x / nshot;
-    const int A = a0 + r % na, C = c0 + r / na, B = D - A - C;
+    const unsigned pos = blockIdx.x >> 3, e = D * 8 + (blockIdx.x & 7);
+    if (pos >= queue.count[e]) return;
+    const unsigned id = queue.list[(long long)e * queue.cap + pos];
+    const unsigned ab = id / queue.nA, cb = ab / queue.nB;
+    const int A = id - ab * queue.nA, B = ab - cb * queue.nB;
+    const int shot = cb / queue.nC, C = cb - shot * queue.nC;
     int zs, zl, xs, xl, ys, yl;
     sweep_axis(w.tz, w.init, g.nzz, sid[3 * shot], zs, zl);
     sweep_axis(w.tx, w.init, g.nxx, sid[3 * shot + 1], xs, xl);
     sweep_axis(w.ty, w.init, g.nyy, sid[3 * shot + 2], ys, yl);
-    if (B < 0 || 8 * B >= xl || 8 * C >= yl || zc * A >= zl) return;
-    float *Ts = T + shot * g.nB;
     const int lane = threadIdx.x;
+    float *Ts = T + shot * g.nB;
     const int len = min(zc, zl - zc * A);      // z cells of this block
     const int nb = min(8, xl - 8 * B), nc = min(8, yl - 8 * C);
     const int z1 = zs + w.tz * (zc * A), x1 = xs + w.tx * (8 * B), y1 = ys + w.ty * (8 * C);
@@ -412,6 +539,7 @@ __global__ __launch_bounds__(64) void fsm_block(float *__restrict__ T,
     // own time and voxels of the step, read one step ahead (no other lane
     // writes them)
     float own = tt[at], vdd = ts[at], vud = ts[at - P], vdu = ts[at - Q], vuu = ts[at - P - Q];
+    bool changed = false;
 #pragma unroll 2
     for (int s = -1; s < len + 14; s++, at++) {
         FsmIn c;
@@ -433,8 +561,9 @@ __global__ __launch_bounds__(64) void fsm_block(float *__restrict__ T,
         c.sen = pmin(suu, vuu);
         c.s = suu;
         const bool on = (unsigned)(at - lo) < (unsigned)len;
-        float res = FAST ? fsm_update_fast(own, c, on, g) : fsm_update_any(own, c, g);
+        float res = FAST ? fsm_update_fast<false>(own, c, on, g) : fsm_update_any(own, c, g);
         res = on ? res : own;
+        if (FULL) changed |= on & !(res == own);
         tt[on ? at : Tile::N] = res;   // the last word takes what is not a cell
         tv = res;
         tev = c.te;
@@ -450,6 +579,16 @@ __global__ __launch_bounds__(64) void fsm_block(float *__restrict__ T,
         vdu = vdu1;
         vuu = vuu1;
         wave_sync();
+    }
+
+    if (FULL) {
+        if (!__any(changed)) return;
+        const bool cx = __any(changed & (x == nb - 1)), cy = __any(changed & (y == nc - 1));
+        // lanes 1 .. 7: the downwind neighbours that read a changed plane
+        const int dA = lane & 1, dB = (lane >> 1) & 1, dC = lane >> 2;
+        if (lane > 0 && lane < 8 && (!dB | cx) && (!dC | cy) && A + dA < queue.nA &&
+            B + dB < queue.nB && C + dC < queue.nC)
+            queue.put_once(shot, A + dA, B + dB, C + dC);
     }
 
     // the block back to memory
@@ -537,11 +676,43 @@ static bool fsm_fast(const st_ctx *ctx, const FsmGeo &g) {
     return lo > 1e-6f && hi < 1e6f && hi < 1000.0f * lo && ctx->smin > 1e-9f && ctx->smax < 1e4f;
 }
 
+// Blocks along the axes and most blocks of one residue of shot + B on the
+// diagonals of a box of nA x nB x nC blocks, for all shots together.
+static void fsm_diagonals(int nA, int nB, int nC, int nshot, std::vector<unsigned> &most) {
+    most.assign(nA + nB + nC - 2, 0);
+    for (int D = 0; D < (int)most.size(); D++) {
+        long long on[8] = {};   // blocks per residue of B
+        for (int B = std::max(0, D - (nA - 1) - (nC - 1)); B <= std::min(D, nB - 1); B++) {
+            const int r = D - B;
+            on[B & 7] += std::min(r, nA - 1) - std::max(0, r - (nC - 1)) + 1;
+        }
+        for (int e = 0; e < 8; e++) {
+            long long n = 0;
+            for (int t = 0; t < 8; t++) n += on[t] * ((nshot + 7 - ((e - t) & 7)) / 8);
+            most[D] = (unsigned)std::max<long long>(most[D], n);
+        }
+    }
+}
+
 // The sixteen sweeps of nshot shots (padded volumes T, source nodes dsid on
-// the device and hsid on the host) on one stream.
+// the device and hsid on the host) on one stream.  A launch per diagonal has
+// as many workgroups as its lists could hold.
 template <int LZ>
 static void fsm_sweeps(hipStream_t st, bool fast, float *T, const float *S, const int *dsid,
-                       const int *hsid, int nshot, const FsmGeo &g) {
+                       const int *hsid, int nshot, const FsmGeo &g, DevBuf &lists) {
+    FsmQueue q{};
+    std::vector<unsigned> most;
+    const int mA = (g.nzz - 1 + LZ - 1) / LZ, mB = (g.nxx + 6) / 8, mC = (g.nyy + 6) / 8;
+    const size_t nD = mA + mB + mC - 2, blocks = (size_t)mA * mB * mC * nshot;
+    ST_REQUIRE(blocks < (1ull << 31), ST_ERR_ARG, "too many blocks for one batch of the sweeps");
+    fsm_diagonals(mA, mB, mC, nshot, most);
+    q.cap = *std::max_element(most.begin(), most.end());
+    const size_t nz = blocks + 16 * nD * 8;   // flags and counts, zero at first
+    lists.reserve(sizeof(unsigned) * (nz + nD * 8 * q.cap));
+    q.flag = lists.as<unsigned>();
+    q.count = q.flag + blocks;
+    q.list = q.flag + nz;
+    ST_HIP(hipMemsetAsync(lists.ptr, 0, sizeof(unsigned) * nz, st));
     for (int pass = 0; pass < 2; pass++) {
         for (int d = 0; d < 8; d++) {
             const FsmSweep w{kDirs[d][0], kDirs[d][1], kDirs[d][2], pass == 0 ? 1 : 0};
@@ -558,20 +729,27 @@ static void fsm_sweeps(hipStream_t st, bool fast, float *T, const float *S, cons
             }
             const int nA0 = (len[0] + LZ - 1) / LZ;
             const int zc = (len[0] + nA0 - 1) / nA0;   // chunks of equal length
-            const int nA = (len[0] + zc - 1) / zc, nB = (len[1] + 7) / 8, nC = (len[2] + 7) / 8;
-            for (int D = 0; D < nA + nB + nC - 2; D++) {
-                const int a0 = std::max(0, D - (nB - 1) - (nC - 1)), a1 = std::min(nA - 1, D);
-                const int c0 = std::max(0, D - (nB - 1) - (nA - 1)), c1 = std::min(nC - 1, D);
-                const int na = a1 - a0 + 1, nc = c1 - c0 + 1;
-                const dim3 grid((unsigned)(na * nc * nshot));
-                if (fast)
-                    hipLaunchKernelGGL((fsm_block<LZ, true>), grid, dim3(64), 0, st, T, S, dsid,
-                                       nshot, g, w, zc, D, a0, na, c0);
-                else
-                    hipLaunchKernelGGL((fsm_block<LZ, false>), grid, dim3(64), 0, st, T, S, dsid,
-                                       nshot, g, w, zc, D, a0, na, c0);
+            q.nA = (len[0] + zc - 1) / zc;
+            q.nB = (len[1] + 7) / 8;
+            q.nC = (len[2] + 7) / 8;
+            q.sweep = d + 1;
+            if (!w.init) {
+                const dim3 grid((unsigned)(((long long)len[0] * len[1] + 255) / 256),
+                                (unsigned)q.nC, (unsigned)nshot);
+                hipLaunchKernelGGL(fast ? fsm_test<true> : fsm_test<false>, grid, dim3(256), 0, st,
+                                   T, S, g, w, zc, q);
             }
+            const long long nb = (long long)q.nA * q.nB * q.nC * nshot;
+            hipLaunchKernelGGL(fsm_list, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, st, dsid,
+                               nshot, g, w, zc, q);
+            fsm_diagonals(q.nA, q.nB, q.nC, nshot, most);
+            const auto walk = fast ? (w.init ? fsm_block<LZ, true, false> : fsm_block<LZ, true, true>)
+                                   : (w.init ? fsm_block<LZ, false, false> : fsm_block<LZ, false, true>);
+            for (int D = 0; D < (int)most.size(); D++)
+                hipLaunchKernelGGL(walk, dim3(most[D] * 8), dim3(64), 0, st, T, S, dsid, g, w, zc, D,
+                                   q);
             ST_HIP(hipGetLastError());
+            q.count += nD * 8;
         }
     }
 }
@@ -599,7 +777,8 @@ double fsm_batch(st_ctx *ctx, const float *dsrc, const float *hsrc, int nshot, c
                        dsid, nshot, g);
     ST_HIP(hipGetLastError());
     const bool fast = fsm_fast(ctx, g);
-    fsm_sweeps<kFsmZ>(ctx->stream, fast, T, S, dsid, hsid.data(), nshot, g);
+    fsm_sweeps<kFsmZ>(ctx->stream, fast, T, S, dsid, hsid.data(), nshot, g,
+                      ctx->fsm_lists);
     ST_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
     ST_HIP(hipEventSynchronize(ctx->ev[3]));
     float ms = 0.f;

@@ -202,6 +202,7 @@ struct st_ctx {
     st::DevBuf counters;               // list counts, stats
     st::DevBuf wstats;                 // per-wave FIM statistics slots
     st::DevBuf fsm_S, fsm_sid;         // sweeping solver: padded slowness, source nodes
+    st::DevBuf fsm_lists;              // flags, counts and lists of its blocks
     st::DevBuf pod_T, pod_stamp, pod_list, pod_counts, pod_nit;   // Podvin
     bool fsm_valid = false;            // fsm_S matches the model
     st::DevBuf src, rcv, picks, scratch;
