@@ -3,7 +3,10 @@
 #include <chrono>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <mutex>
+#include <system_error>
+#include <thread>
 
 #include "st_common.hpp"
 
@@ -271,6 +274,9 @@ int st_ctx_destroy(st_ctx *ctx) {
                     &ctx->picks, &ctx->scratch, &ctx->keys, &ctx->kmin, &ctx->judge, &ctx->pred,
                     &ctx->tkeys, &ctx->xfaces})
         b->release();
+    if (ctx->rb_pinned) (void)hipHostFree(ctx->rb_pinned);
+    for (auto &e : ctx->rb_ev)
+        if (e) (void)hipEventDestroy(e);
     for (auto &e : ctx->ev)
         if (e) (void)hipEventDestroy(e);
     if (ctx->host_pinned) (void)hipHostFree(ctx->host_pinned);
@@ -331,6 +337,80 @@ static void upload_points(st_ctx *ctx, const float *src_xyz, int nshot, const fl
     if (nrcv)
         ST_HIP(hipMemcpyAsync(ctx->rcv.ptr, rcv_xyz, sizeof(float) * 3 * nrcv,
                               hipMemcpyHostToDevice, ctx->stream));
+}
+
+constexpr size_t kReadBackMin = 8u << 20;
+
+// A device result to host memory at dst, queued on the context's stream; done
+// when the stream is.  Large results to ordinary memory are done on return:
+// the runtime's copy moves them with one host thread, which also takes the
+// page faults of a fresh array; here four threads move chunks from pinned
+// slots, each its own slots, while the next chunks arrive.  The slots (8 MiB)
+// stay with the context.  Time of the read-back alone, before and now: 38 MB
+// 3.66 and 1.40 ms, 17 MB 1.02 and 0.61, 8.5 MB 0.57 and 0.37, 4.2 MB 0.28 and
+// 0.22 -- where the slots' allocation costs the first call 0.45 ms, so the
+// line lies at kReadBackMin.
+static void read_back(st_ctx *ctx, void *dst, const void *src, size_t bytes) {
+    constexpr size_t chunk = 1 << 20;
+    constexpr int slots = st_ctx::kReadBackSlots, workers = 4;
+    bool plain = bytes < kReadBackMin;
+    if (!plain) {   // pinned, managed and device memory go the direct way
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, dst) != hipSuccess)
+            (void)hipGetLastError();
+        else
+            plain = at.type != hipMemoryTypeUnregistered;
+    }
+    if (plain) {
+        ST_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ctx->stream));
+        return;
+    }
+    if (!ctx->rb_pinned) {
+        for (auto &e : ctx->rb_ev)
+            if (!e) ST_HIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+        ST_HIP(hipHostMalloc(&ctx->rb_pinned, chunk * slots, hipHostMallocDefault));
+    }
+    const size_t n = (bytes + chunk - 1) / chunk;
+    char *const pin = static_cast<char *>(ctx->rb_pinned);
+    auto size = [&](size_t c) { return std::min(chunk, bytes - c * chunk); };
+    auto fetch = [&](size_t c) {   // chunk c to its slot
+        ST_HIP(hipMemcpyAsync(pin + c % slots * chunk, static_cast<const char *>(src) + c * chunk,
+                              size(c), hipMemcpyDeviceToHost, ctx->stream));
+        ST_HIP(hipEventRecord(ctx->rb_ev[c % slots], ctx->stream));
+    };
+    // worker w moves the chunks of the slots w, w + workers, ...
+    auto work = [&](int w) {
+        ST_HIP(hipSetDevice(ctx->device));
+        for (size_t c = w; c < n; c += workers) {
+            ST_HIP(hipEventSynchronize(ctx->rb_ev[c % slots]));
+            std::memcpy(static_cast<char *>(dst) + c * chunk, pin + c % slots * chunk, size(c));
+            if (c + slots < n) fetch(c + slots);
+        }
+    };
+    static_assert(slots % workers == 0, "a slot belongs to one worker");
+    std::exception_ptr failed[workers];
+    auto guarded = [&](int w) {
+        try {
+            work(w);
+        } catch (...) {
+            failed[w] = std::current_exception();
+        }
+    };
+    for (size_t c = 0; c < std::min<size_t>(slots, n); c++) fetch(c);
+    std::thread other[workers];
+    int started = 1;
+    try {
+        for (; started < workers; started++) other[started] = std::thread(guarded, started);
+    } catch (const std::system_error &) {   // no more threads: this one does the rest
+    }
+    guarded(0);
+    for (int w = started; w < workers; w++) guarded(w);
+    for (int w = 1; w < started; w++) other[w].join();
+    for (auto &f : failed)
+        if (f) {
+            (void)hipStreamSynchronize(ctx->stream);   // no copy into the slots is left
+            std::rethrow_exception(f);
+        }
 }
 
 // The sweeping solver's padded slowness (rebuilt after a model change) and
@@ -474,8 +554,7 @@ static void solve_impl(st_ctx *ctx, const float *src_xyz, int nshot, const float
                              ctx->nz, ctx->dx, ctx->dy, ctx->dz, B, g.nbx, g.nby);
         if (T_out) {
             launch_extract(ctx, ctx->scratch.as<float>(), nb, B);
-            ST_HIP(hipMemcpyAsync(T_out + (long long)b0 * npts, ctx->scratch.ptr,
-                                  sizeof(float) * npts * nb, hipMemcpyDeviceToHost, ctx->stream));
+            read_back(ctx, T_out + (long long)b0 * npts, ctx->scratch.ptr, sizeof(float) * npts * nb);
             ST_HIP(hipStreamSynchronize(ctx->stream));
         }
         if (!bad.empty()) {
@@ -503,9 +582,8 @@ static void solve_impl(st_ctx *ctx, const float *src_xyz, int nshot, const float
             if (T_out) {
                 launch_extract(ctx, ctx->scratch.as<float>(), k, B);
                 for (int q = 0; q < k; q++)
-                    ST_HIP(hipMemcpyAsync(T_out + (long long)(b0 + bad[q]) * npts,
-                                          ctx->scratch.as<float>() + q * npts, sizeof(float) * npts,
-                                          hipMemcpyDeviceToHost, ctx->stream));
+                    read_back(ctx, T_out + (long long)(b0 + bad[q]) * npts,
+                              ctx->scratch.as<float>() + q * npts, sizeof(float) * npts);
                 ST_HIP(hipStreamSynchronize(ctx->stream));
             }
         }
@@ -666,9 +744,8 @@ int st_fsm_solve(st_ctx *ctx, const float *src_xyz, int nshot, const float *rcv_
                           ctx->picks.as<float>() + (long long)b0 * nrcv);
             if (T_out) {
                 fsm_crop_volumes(ctx, ctx->scratch.as<float>(), nb);
-                ST_HIP(hipMemcpyAsync(T_out + (long long)b0 * npts, ctx->scratch.ptr,
-                                      sizeof(float) * npts * nb, hipMemcpyDeviceToHost,
-                                      ctx->stream));
+                read_back(ctx, T_out + (long long)b0 * npts, ctx->scratch.ptr,
+                          sizeof(float) * npts * nb);
                 ST_HIP(hipStreamSynchronize(ctx->stream));
             }
         }
@@ -706,9 +783,8 @@ int st_podvin_solve(st_ctx *ctx, const float *src_xyz, int nshot, const float *r
                              ctx->picks.as<float>() + (long long)b0 * nrcv);
             if (T_out) {
                 podvin_crop_volumes(ctx, ctx->scratch.as<float>(), nb);
-                ST_HIP(hipMemcpyAsync(T_out + (long long)b0 * npts, ctx->scratch.ptr,
-                                      sizeof(float) * npts * nb, hipMemcpyDeviceToHost,
-                                      ctx->stream));
+                read_back(ctx, T_out + (long long)b0 * npts, ctx->scratch.ptr,
+                          sizeof(float) * npts * nb);
                 ST_HIP(hipStreamSynchronize(ctx->stream));
             }
         }
@@ -831,8 +907,7 @@ static void forward_impl(st_ctx *ctx, const float *src_xyz, int nshot, const flo
     tomo_reset(ctx, true);
     // one batch: solve, pick, trace its rays; the travel times to T_out
     auto to_host = [&](int b0, int nb) {
-        ST_HIP(hipMemcpyAsync(T_out + (long long)b0 * npts, ctx->scratch.ptr,
-                              sizeof(float) * npts * nb, hipMemcpyDeviceToHost, ctx->stream));
+        read_back(ctx, T_out + (long long)b0 * npts, ctx->scratch.ptr, sizeof(float) * npts * nb);
         ST_HIP(hipStreamSynchronize(ctx->stream));
     };
     const float *drcv = ctx->rcv.as<float>();

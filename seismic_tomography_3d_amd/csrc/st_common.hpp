@@ -205,6 +205,9 @@ struct st_ctx {
     st::DevBuf fsm_lists;              // flags, counts and lists of its blocks
     st::DevBuf pod_T, pod_stamp, pod_list, pod_counts, pod_nit;   // Podvin
     bool fsm_valid = false;            // fsm_S matches the model
+    static constexpr int kReadBackSlots = 8;
+    void *rb_pinned = nullptr;         // pinned slots of large read-backs, an event each
+    hipEvent_t rb_ev[kReadBackSlots] = {};
     st::DevBuf src, rcv, picks, scratch;
     st::DevBuf keys, kmin, judge, pred;   // warm-start state
     st::DevBuf tkeys;                  // arrival-ordering keys (2 x batch x nblk)
