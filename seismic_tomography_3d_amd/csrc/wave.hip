@@ -736,21 +736,24 @@ void wave_shots(st_ctx *ctx, const float *wavelet, int nt, const float *src_xyz,
     }
     G = std::min(G, nshot);
     G = (int)std::max<long long>(1, std::min<long long>(G, (24LL << 30) / (8 * N)));
-    // planes per workgroup: the chunk length whose busiest CU is done first.
-    // A chunk of y planes costs y + 4 plane times (the ring's first nine
-    // planes are read before the first step), a plane time shared by three
-    // resident workgroups is the unit, and two or one of them leave a tenth
-    // or a third of the CU idle.  One shot of 141 x 121 x 81 cells and 50
-    // layer cells (45 tiles, 213 planes): 32 planes (the former rule's
-    // minimum, 1.2 workgroups per CU) 48 ms for 801 steps, 20: 35, 16: 33,
-    // 13 (765 workgroups, chosen) 30, 10: 38, 8: 34.
+    // planes per workgroup: the chunk length that is done first.  Three
+    // workgroups fit a CU, so they run in rounds of 3 ncu; a last round with
+    // two or one left per CU takes 0.73 or 0.5 of a full one's time.  A chunk
+    // of y planes costs y + 2 plane times (the ring's first planes are read
+    // before the first step).  Measured, us per step at y planes:
+    //   45 tiles, 213 planes: 32 (the former rule's least) 60, 20: 43, 16: 42,
+    //     13 (chosen: 765 workgroups) 38, 10: 48, 8: 43
+    //   175 tiles, 593 planes: 100: 492, 85: 467, 64: 478, 48: 430, 46
+    //     (chosen: 2,275) 422, 32: 443, 24: 436, 16: 440
     int ncu = 0;
     ST_HIP(hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, ctx->device));
     long long best = LLONG_MAX;
     for (int y = std::min(4, nyi); y <= nyi; y++) {
-        const long long per_cu = (G * tiles * ((nyi + y - 1) / y) + ncu - 1) / ncu;
-        const long long cost = per_cu * (y + 4) * (per_cu == 1 ? 15 : per_cu == 2 ? 11 : 10);
-        if (cost <= best) {
+        const long long wg = G * tiles * ((nyi + y - 1) / y), left = wg % (3 * ncu);
+        const int part[4] = {0, 15, 22, 30};   // of a round, in thirtieths
+        const long long cost =
+            (y + 2) * (30 * (wg / (3 * ncu)) + part[(left + ncu - 1) / ncu]);
+        if (cost < best) {
             best = cost;
             a.ychunk = y;
         }
