@@ -319,7 +319,7 @@ int st_acoustic_set_model(st_ctx *ctx, const float *vel, int nx, int ny, int nz,
  * then per step applyWavelet, wavePropagation, wavefieldUpdate,
  * buildSeismogram).  Sources and receivers sit at cell (int)(p / d) + nb
  * per axis and must lie in the model.  group = shots advanced together
- * (0 = automatic: enough to fill the device; each holds three wavefields).
+ * (0 = automatic: enough to fill the device; each holds two wavefields).
  * seis (nullable):
  * [nshot][nrec][nt] (the reference's seismogram[t + r nt] per shot);
  * ufut_last (nullable): the last shot's final U_fut (nyy*nxx*nzz padded

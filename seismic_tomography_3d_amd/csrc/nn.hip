@@ -1,7 +1,7 @@
 // nn.hip -- hand-written training and inference kernels of the warm-start
-// network: BF16 MFMA GEMM with FP32 accumulation, 3D im2col / col2im,
-// average pooling, nearest upsampling, channel concat, bias/ReLU, MSE loss
-// and Adam.  Activations are channels-last [sample][z][y][x][c], voxel
+// network: BF16 MFMA GEMM with FP32 accumulation, 3D convolutions forward and
+// backward without an im2col matrix, average pooling, nearest upsampling,
+// channel concat, bias/ReLU, MSE loss and Adam.  Activations are channels-last [sample][z][y][x][c], voxel
 // v = x + n*(y + n*z) on an n^3 cube.
 #include <type_traits>
 
