@@ -488,14 +488,16 @@ __global__ __launch_bounds__(256) void conv3d_bwd_x(const unsigned short *__rest
 // lanes x 4 BF16, lane = m + 16 q holding W[tap, c = 16 ct + m, n = 16 k + 4 q
 // + i]; zero past cin and cout.  W16 is [tap*cin + c][cout].
 __global__ void pack_conv_bwd(const unsigned short *__restrict__ W16,
-                              unsigned short *__restrict__ Wb, int taps, int cin, int cout, int kc,
-                              int ctt) {
-    const int tot = taps * kc * ctt * 256;
+                              unsigned short *__restrict__ Wb, BwdPack p) {
+    const BwdPack::Layer l = p.l[blockIdx.y];
+    const int kc = (l.cout + 15) / 16, ctt = (l.cin + 15) / 16, tot = l.taps * kc * ctt * 256;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < tot; i += gridDim.x * blockDim.x) {
         const int u = i & 3, lane = (i >> 2) & 63, f = i >> 8;
         const int ct = f % ctt, k = (f / ctt) % kc, tap = f / (ctt * kc);
         const int c = 16 * ct + (lane & 15), n = 16 * k + 4 * (lane >> 4) + u;
-        Wb[i] = c < cin && n < cout ? W16[((long long)tap * cin + c) * cout + n] : (unsigned short)0;
+        Wb[l.to + i] = c < l.cin && n < l.cout
+                           ? W16[l.from + ((long long)tap * l.cin + c) * l.cout + n]
+                           : (unsigned short)0;
     }
 }
 
@@ -598,6 +600,18 @@ __global__ __launch_bounds__(256) void conv3d_bwd_w(const float *__restrict__ X,
             }
         }
         __syncthreads();
+    }
+    if (KS == 1) {   // the four waves' sums of the same weights, one addition each
+        static_assert(KS != 1 || (CT == 1 && sizeof(sX) >= 4096), "room for the sums");
+        float *red = reinterpret_cast<float *>(sX);
+#pragma unroll
+        for (int r = 0; r < 4; r++) red[tid * 4 + r] = acc[0][0][r];
+        __syncthreads();
+        const int l = tid >> 2, c = c0 + 4 * (l >> 4) + (tid & 3), n = n0 + (l & 15);
+        if (c < cin && n < cout)
+            atomicAdd(&dW[(long long)c * cout + n],
+                      (red[tid] + red[256 + tid]) + (red[512 + tid] + red[768 + tid]));
+        return;
     }
 #pragma unroll
     for (int i = 0; i < TW; i++) {
@@ -904,14 +918,22 @@ long long conv_bwd_packed_size(int ksz, int cin, int cout) {
     return (long long)ksz * ksz * ksz * ((cout + 15) / 16) * ((cin + 15) / 16) * 256;
 }
 
-void conv_backward_input(hipStream_t st, const unsigned short *D, const unsigned short *W16,
-                         unsigned short *Wb, float *dX, int ns, int e, int cin, int cout, int ksz) {
+void pack_conv_backward(hipStream_t st, const unsigned short *W16, unsigned short *Wb,
+                        const BwdPack &p) {
+    long long most = 0;
+    for (int i = 0; i < p.n; i++)
+        most = std::max(most, (long long)p.l[i].taps * ((p.l[i].cout + 15) / 16) *
+                                  ((p.l[i].cin + 15) / 16) * 256);
+    hipLaunchKernelGGL(pack_conv_bwd, dim3(blocks_for(most), p.n), dim3(256), 0, st, W16, Wb, p);
+    ST_HIP(hipGetLastError());
+}
+
+void conv_backward_input(hipStream_t st, const unsigned short *D, const unsigned short *Wb,
+                         float *dX, int ns, int e, int cin, int cout, int ksz) {
     const int kc = (cout + 15) / 16, ctt = (cin + 15) / 16, ct = bwd_tiles(cin);
-    const int taps = ksz * ksz * ksz, nb = bwd_bricks(ns, e);
+    const int nb = bwd_bricks(ns, e);
     ST_REQUIRE(ctt % ct == 0, ST_ERR_ARG, "conv channels");
     if (nb == 0) return;
-    hipLaunchKernelGGL(pack_conv_bwd, dim3(blocks_for(conv_bwd_packed_size(ksz, cin, cout))),
-                       dim3(256), 0, st, W16, Wb, taps, cin, cout, kc, ctt);
     const dim3 g(nb, ctt / ct), b(256);
 #define ST_BWD_X(KS, NP, CT)                                                                      \
     if (ksz == KS && kc * 16 == NP && ct == CT) {                                                 \
@@ -938,9 +960,10 @@ void conv_backward_weight(hipStream_t st, const float *X, const unsigned short *
     ST_REQUIRE(ctt % ct == 0, ST_ERR_ARG, "conv channels");
     if (nb == 0) return;
     // two workgroups per CU over all channel groups, each adding its sums once;
-    // fewer for the 1^3 head, whose few sums would queue (512: 113 us at 262,144
-    // voxels)
-    const int gx = std::max(1, std::min(nb, (ksz == 1 ? 64 : 512) / (cchunks * nt)));
+    // fewer for the 1^3 head, whose workgroups all add to the same few weights
+    // (16 of them, 262,144 voxels: 64 / 128 / 256 / 512 workgroups 70 / 38 / 29 /
+    // 35 us; 74 with 64 and an addition per wave)
+    const int gx = std::max(1, std::min(nb, (ksz == 1 ? 256 : 512) / (cchunks * nt)));
     const dim3 g(gx, cchunks * nt), b(256);
 #define ST_BWD_W(KS, CT)                                                                          \
     if (ksz == KS && ct == CT) {                                                                  \

@@ -53,11 +53,20 @@ void pack_conv_weights(hipStream_t st, const unsigned short *W16, unsigned short
 void conv_forward(hipStream_t st, const float *X, const unsigned short *Wp, const float *bias,
                   float *Y, int ns, int e, int cin, int cout, int ksz, bool relu);
 // gradients of the same convolution from D, the masked output gradient in
-// BF16: dX written (Wb: conv_bwd_packed_size entries of scratch for the
-// re-ordered weights W16), dW [tap*cin + c][cout] added to
+// BF16: dX written (Wb: the layer's weights as pack_conv_backward re-orders
+// them, conv_bwd_packed_size entries), dW [tap*cin + c][cout] added to
 long long conv_bwd_packed_size(int ksz, int cin, int cout);
-void conv_backward_input(hipStream_t st, const unsigned short *D, const unsigned short *W16,
-                         unsigned short *Wb, float *dX, int ns, int e, int cin, int cout, int ksz);
+struct BwdPack {   // layers re-ordered by one launch: from, to in entries
+    struct Layer {
+        long long from, to;
+        int taps, cin, cout;
+    } l[16];
+    int n;
+};
+void pack_conv_backward(hipStream_t st, const unsigned short *W16, unsigned short *Wb,
+                        const BwdPack &p);
+void conv_backward_input(hipStream_t st, const unsigned short *D, const unsigned short *Wb,
+                         float *dX, int ns, int e, int cin, int cout, int ksz);
 void conv_backward_weight(hipStream_t st, const float *X, const unsigned short *D, float *dW,
                           int ns, int e, int cin, int cout, int ksz);
 // the forward pass with the input the concatenation [X0 (C0 channels, nearest-

@@ -170,13 +170,13 @@ static void net_alloc_batch(Net &n, int ns, bool train) {
     F(n.d_a4, v2 * 32); F(n.d_t16, v2 * 32); F(n.d_cat3, v4 * 128); F(n.d_a7, v8 * 64);
     F(n.d_a5, v4 * 64); F(n.d_t8, v4 * 64); F(n.d_p3, v8 * 64); F(n.d_p2, v4 * 32);
     F(n.d_a3, v2 * 32); F(n.d_p1, v2 * 16); F(n.d_a1, v1 * 16); F(n.d_in, v1 * kIn);
-    long long ymax = 0, wmax = 0;
+    long long ymax = 0, wsum = 0;
     for (auto &c : n.L) {
         ymax = std::max(ymax, cube(n.nc / c.res_div) * ns * c.cout);
-        wmax = std::max(wmax, nn::conv_bwd_packed_size(c.ksz, c.cin, c.cout));
+        wsum += nn::conv_bwd_packed_size(c.ksz, c.cin, c.cout);
     }
     n.d16.reserve(sizeof(unsigned short) * ymax);
-    n.wb.reserve(sizeof(unsigned short) * wmax);
+    n.wb.reserve(sizeof(unsigned short) * wsum);
     n.lossacc.reserve(64);
     n.tcap = ns;
 }
@@ -208,6 +208,14 @@ static void net_pack(st_ctx *ctx, Net &n) {
     n.pver = n.wver;
 }
 
+// where a layer's weights start among those re-ordered for the backward pass
+static long long packed_at(const Net &n, int li) {
+    long long at = 0;
+    for (int i = 0; i < li; i++)
+        at += nn::conv_bwd_packed_size(n.L[i].ksz, n.L[i].cin, n.L[i].cout);
+    return at;
+}
+
 // one convolution backward: dY -> dW, db (+=), dX (written)
 static void conv_bwd(st_ctx *ctx, Net &n, int li, const float *X, const float *Y, const float *dY,
                      float *dX, int ns) {
@@ -219,8 +227,8 @@ static void conv_bwd(st_ctx *ctx, Net &n, int li, const float *X, const float *Y
     nn::conv_backward_weight(ctx->stream, X, d16, n.g.as<float>() + c.ow, ns, e, c.cin, c.cout,
                              c.ksz);
     if (dX)
-        nn::conv_backward_input(ctx->stream, d16, n.w16.as<unsigned short>() + c.ow,
-                                n.wb.as<unsigned short>(), dX, ns, e, c.cin, c.cout, c.ksz);
+        nn::conv_backward_input(ctx->stream, d16, n.wb.as<unsigned short>() + packed_at(n, li), dX,
+                                ns, e, c.cin, c.cout, c.ksz);
 }
 
 __global__ void add_into(float *__restrict__ y, const float *__restrict__ x, long long n) {
@@ -304,6 +312,12 @@ static void net_backward(st_ctx *ctx, Net &n, int ns, const float *target, const
     const long long V1 = cube(e1) * ns, V2 = cube(e2) * ns, V4 = cube(e4) * ns;
     ST_HIP(hipMemsetAsync(n.g.ptr, 0, sizeof(float) * n.nparam, st));
     ST_HIP(hipMemsetAsync(n.lossacc.ptr, 0, 2 * sizeof(double), st));
+    nn::BwdPack pack{};
+    for (const Conv &c : n.L) {
+        pack.l[pack.n] = {c.ow, packed_at(n, pack.n), c.ksz * c.ksz * c.ksz, c.cin, c.cout};
+        pack.n++;
+    }
+    nn::pack_conv_backward(st, n.w16.as<unsigned short>(), n.wb.as<unsigned short>(), pack);
     nn::mse_loss(st, n.out.as<float>(), target, mask, n.d_out.as<float>(), n.lossacc.as<double>(), V1,
                  n.under_weight);
     conv_bwd(ctx, n, 9, n.a10.as<float>(), n.out.as<float>(), n.d_out.as<float>(), n.d_a10.as<float>(), ns);
