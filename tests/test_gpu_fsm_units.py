@@ -1,0 +1,34 @@
+"""Accurate_FSM on the device over units of spacing and slowness: 25 m cells,
+the coarser ones of crustal models, where 2D roots beside the source have
+negative arguments and the method's NaN decides.  Travel times must equal the
+oracle's in every bit.
+"""
+import numpy as np
+import pytest
+
+import oracle_lib as orc
+
+pytestmark = pytest.mark.gpu
+
+
+def _equal_oracle(ctx, shape, d, slow, seed):
+    nx, ny, nz = shape
+    rng = np.random.default_rng(seed)
+    s = rng.uniform(*slow, (ny, nx, nz)).astype(np.float32)
+    ctx.set_model(s, *d)
+    L = ((np.array(shape) - 1) * np.array(d)).astype(np.float32)
+    src = np.concatenate([rng.uniform(0, 1, (4, 3)), [[0, 0, 0], [1, 1, 1], [0.5, 0.5, 0.5]]]) * L
+    src = np.minimum(src.astype(np.float32), L)
+    _, T, _ = ctx.fsm_solve(src, np.zeros((1, 3), np.float32), return_T=True)
+    T0 = np.empty((ny, nx, nz), np.float32)
+    for i, p in enumerate(src):
+        orc.oracle().or_fsm(orc.P(s), nx, ny, nz, *d, float(p[0]), float(p[1]), float(p[2]),
+                            orc.P(T0))
+        assert np.array_equal(T[i], T0), (i, T[i].min(), np.abs(T[i] - T0).max())
+
+
+@pytest.mark.parametrize("v", [1500.0, 3000.0, 6000.0, 12500.0])
+@pytest.mark.parametrize("h", [25.0, 50.0, 100.0, 130.0, 200.0, 250.0, 500.0, 1000.0])
+def test_spacings_and_speeds(ctx, h, v):
+    _equal_oracle(ctx, (21, 19, 17), (h, h, h), (1 / v, 1 / v + 1e-12), int(h + v))
+    _equal_oracle(ctx, (21, 19, 17), (h, 0.8 * h, 0.5 * h), (0.9 / v, 1.1 / v), int(h + v))
