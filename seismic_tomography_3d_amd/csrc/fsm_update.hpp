@@ -155,11 +155,11 @@ __device__ float fsm_update_any(float T, const FsmIn &c, const FsmGeo &g) {
 // PRUNE, with lim the least of the cell's time and the 1D operators:
 // * t3D is at least the weighted mean of its arms (its root is not negative
 //   and rounding is monotone), a linear form of the seven upwind times; above
-//   lim by more than rounding (2^-17 of the times) it is ruled out;
+//   lim by more than rounding (2^-17 of lim and the times) it is ruled out;
 // * a 2D operator is at least its diagonal time plus the slowness times the
 //   lesser spacing (its root term is concave in the difference of the two
 //   axis times, with the spacings' values at the ends of the admitted range);
-//   with 1 % of that term and 2^-16 of lim for rounding, at or above lim it
+//   with 1 % of that term and the same share for rounding, at or above lim it
 //   is ruled out -- unless the 3D operator is in play, whose condition reads
 //   the 2D times.
 // A NaN left out offers nothing but may have kept others from lowering the
@@ -187,11 +187,11 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
         l3 = __builtin_fmaf(g.wen, c.ten, l3);
         l3 = __builtin_fmaf(g.wnv, c.tnv, l3);
         const float big = pmax(pmax(latest, c.tnve), pmax(c.tev, pmax(c.ten, c.tnv)));
-        try3 = on & (t1D > latest) & (l3 < __builtin_fmaf(big + lim, 7.6293945e-6f, lim));
-        const float far2 = lim * 1.0000153f;
-        pxz = try3 | (on & (__builtin_fmaf(c.sve, g.dmin, c.tev) < far2));
-        pyz = try3 | (on & (__builtin_fmaf(c.svn, g.dmin, c.tnv) < far2));
-        pxy = try3 | (on & (__builtin_fmaf(c.sen, g.dmin, c.ten) < far2));
+        const float far = __builtin_fmaf(big + lim, 7.6293945e-6f, lim);
+        try3 = on & (t1D > latest) & (l3 < far);
+        pxz = try3 | (on & (__builtin_fmaf(c.sve, g.dmin, c.tev) < far));
+        pyz = try3 | (on & (__builtin_fmaf(c.svn, g.dmin, c.tnv) < far));
+        pxy = try3 | (on & (__builtin_fmaf(c.sen, g.dmin, c.ten) < far));
     }
     float xz = 1e6f, yz = 1e6f, xy = 1e6f, t3D = 1e6f;
     if (!PRUNE || __any(pxz)) {

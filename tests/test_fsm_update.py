@@ -27,3 +27,8 @@ def compare(tmp_path_factory):
 @pytest.mark.parametrize("draws,per", [(0, 10000), (400, 4000)])   # ordinary units, the whole range
 def test_walk_equals_general_form(compare, draws, per):
     compare("walk", draws, per, 1)
+
+
+@pytest.mark.parametrize("draws,per", [(0, 10000), (400, 4000)])
+def test_test_lowers_what_the_general_form_lowers(compare, draws, per):
+    compare("test", draws, per, 2)
