@@ -61,11 +61,13 @@ inline FsmGeo fsm_geometry(int nx, int ny, int nz, float dx, float dy, float dz)
 
 // Whether the FAST update's ranges hold: spacings and their squares far from
 // under- and overflow and within a factor of 1000 of each other (the slack of
-// its 2D bound), root arguments 0 or above 2^-102, times of ordinary size.
+// its 2D bound), times of ordinary size, root arguments 0 or of 2^-101 and more:
+// an argument is (s / d)^2 times at least 8 less another number, and where the
+// two cancel, a multiple of 2^-25 of it.
 inline bool fsm_fast(const FsmGeo &g, float slow_min, float slow_max) {
     const float lo = std::min({g.dx, g.dy, g.dz}), hi = std::max({g.dx, g.dy, g.dz});
     return lo > 1e-6f && hi < 1e6f && hi < 1000.0f * lo && slow_min > 1e-9f &&
-           slow_max < 1e4f;
+           slow_min > 1e-11f * hi && slow_max < 1e4f;
 }
 
 // Upwind travel times of a cell (v along z, e along x, n along y and their

@@ -1,7 +1,7 @@
 // The two forms of Accurate_FSM's cell update, built for the host: the short
 // form against the form of the method's code.
 //
-//   fsm_update_host walk|test <draws of units> <neighbourhoods per units> <seed>
+//   fsm_update_host walk|test|roots <draws of units> <neighbourhoods per units> <seed>
 //
 // Units are drawn over the whole range that the short form is admitted for
 // (with 0 draws: a list of ordinary ones).  For each set of units,
@@ -9,8 +9,11 @@
 // passing fronts at a distance of up to 10^5 cells, times at the edges of the
 // operators' ranges to the last bit, and arbitrary ones.  walk: the form of the
 // blocks' walk must equal the general one in every bit; test: the form with
-// operators left out must lower every cell the general one lowers.  Prints what
-// differs and the counts; fails if any does.
+// operators left out must lower every cell the general one lowers; roots: as
+// walk, with units of the least slowness to spacing and one time of each
+// neighbourhood moved to where the argument of the 3D operator's root is a few
+// units of its last place.  Prints what differs and the counts; fails if any
+// does.
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -107,11 +110,37 @@ FsmIn neighbourhood(const Units &u, float &T) {
     return c;
 }
 
+// t2 - t3 of the 3D operator, as the update has them
+float root_argument(const FsmIn &c, const FsmGeo &g) {
+    float ta, tb, tc;
+    fsm_arms(c, ta, tb, tc);
+    const float t2 = 9.0f * c.s * c.s * g.dsum;
+    const float t3 = g.dz2dx2 * (ta - tb) * (ta - tb) + g.dz2dy2 * (tb - tc) * (tb - tc) +
+                     g.dx2dy2 * (ta - tc) * (ta - tc);
+    return t2 - t3;
+}
+
+// Moves tnv, which two arms hold with different signs, until the argument
+// passes zero, and leaves it within three units of there.
+void cancel_root(FsmIn &c, const FsmGeo &g) {
+    if (!(root_argument(c, g) > 0)) return;
+    FsmIn out = c;
+    const float step = c.s * std::min({g.dx, g.dy, g.dz});
+    for (int k = 0; k < 8 && root_argument(out, g) >= 0; k++) out.tnv += step;
+    if (root_argument(out, g) >= 0) return;
+    int a = __float_as_int(c.tnv), b = __float_as_int(out.tnv);
+    while (b - a > 1) {
+        out.tnv = __int_as_float(a + (b - a) / 2);
+        (root_argument(out, g) >= 0 ? a : b) = a + (b - a) / 2;
+    }
+    c.tnv = __int_as_float(std::max(0, a - pick(4)));
+}
+
 }  // namespace
 
 int main(int argc, char **argv) {
     if (argc != 5) return 2;
-    const bool walk = !std::strcmp(argv[1], "walk");
+    const bool roots = !std::strcmp(argv[1], "roots"), walk = roots || !std::strcmp(argv[1], "walk");
     const int draws = std::atoi(argv[2]), per = std::atoi(argv[3]);
     rng.seed((unsigned)std::atoi(argv[4]));
     std::vector<Units> units;
@@ -123,11 +152,12 @@ int main(int argc, char **argv) {
             }
     while ((int)units.size() < draws) {
         Units u;
-        const double mid = logu(1e-6, 1e6), ratio = logu(1, 1000);
+        const double mid = logu(roots ? 1e3 : 1e-6, 1e6), ratio = logu(1, roots ? 2 : 1000);
         float *d[3] = {&u.dx, &u.dy, &u.dz};
         for (float *p : d) *p = (float)(mid * std::pow(ratio, uni(0, 1)));
         u.lo = (float)logu(1e-9, 1e4);
-        u.hi = pick(2) ? u.lo : (float)logu(u.lo, 1e4);
+        if (roots) u.lo = (float)(mid * logu(1e-15, 1e-10));
+        u.hi = roots || pick(2) ? u.lo : (float)logu(u.lo, 1e4);
         if (fsm_fast(fsm_geometry(2, 2, 2, u.dx, u.dy, u.dz), u.lo, u.hi)) units.push_back(u);
     }
     long all = 0, bad = 0;
@@ -135,7 +165,8 @@ int main(int argc, char **argv) {
         const FsmGeo g = fsm_geometry(2, 2, 2, u.dx, u.dy, u.dz);
         for (int k = 0; k < per; k++) {
             float T;
-            const FsmIn c = neighbourhood(u, T);
+            FsmIn c = neighbourhood(u, T);
+            if (roots) cancel_root(c, g);
             const float a = fsm_update_any(T, c, g), b = walk ? fsm_update_fast<false>(T, c, true, g)
                                                              : fsm_update_fast<true>(T, c, true, g);
             all++;

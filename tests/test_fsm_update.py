@@ -32,3 +32,7 @@ def test_walk_equals_general_form(compare, draws, per):
 @pytest.mark.parametrize("draws,per", [(0, 10000), (400, 4000)])
 def test_test_lowers_what_the_general_form_lowers(compare, draws, per):
     compare("test", draws, per, 2)
+
+
+def test_roots_next_to_zero(compare):
+    compare("roots", 2000, 2000, 3)

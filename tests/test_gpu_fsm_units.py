@@ -32,3 +32,16 @@ def _equal_oracle(ctx, shape, d, slow, seed):
 def test_spacings_and_speeds(ctx, h, v):
     _equal_oracle(ctx, (21, 19, 17), (h, h, h), (1 / v, 1 / v + 1e-12), int(h + v))
     _equal_oracle(ctx, (21, 19, 17), (h, 0.8 * h, 0.5 * h), (0.9 / v, 1.1 / v), int(h + v))
+
+
+@pytest.mark.parametrize("d", [(900.0, 1.0, 1.0), (1.0, 1.0, 900.0), (1.0, 30.0, 900.0)])
+def test_spacings_far_apart(ctx, d):
+    _equal_oracle(ctx, (21, 19, 17), d, (2e-4, 7e-4), 1)
+    _equal_oracle(ctx, (5, 7, 90), d, (2e-4, 7e-4), 2)
+
+
+@pytest.mark.parametrize("d,s", [(9e5, 2e-9),      # root arguments too small for the short form
+                                 (9e5, 9.1e-6),    # just large enough
+                                 (20.0, 2e-9)])
+def test_slownesses_small_against_the_spacing(ctx, d, s):
+    _equal_oracle(ctx, (21, 19, 17), (d, 0.9 * d, 0.8 * d), (s, 1.01 * s), 3)
