@@ -559,7 +559,7 @@ __global__ __launch_bounds__(256) void conv3d_bwd_w(const float *__restrict__ X,
             const int hx = hv % HX, row = hv / HX;
             const int x = 8 * bx + hx - HF, y = 4 * by + row % HY - HF, z = 4 * bz + row / HY - HF;
             unsigned short h[4] = {0, 0, 0, 0};
-            if (x >= 0 && y >= 0 && z >= 0 && x < e && y < e && z < e) {
+            if (x >= 0 && y >= 0 && z >= 0 && x < e && y < e && z < e && n0 + n < cout) {
                 const unsigned short *p =
                     D + (base + x + (long long)e * (y + (long long)e * z)) * cout + n0 + n;
                 if ((cout & 3) == 0) {
