@@ -24,7 +24,8 @@
 // in any order, and operators that cannot lower the cell are left out:
 // * one none of whose times changed in the last step gave the same arrival
 //   when they last changed (the cell was active then), and the cell has kept
-//   the minimum (from the start on, where unreached times offer nothing);
+//   the minimum (from the start on, where unreached times offer nothing: no
+//   time is above them but that of a source that starts no front);
 // * arrivals of the form X + root are not below X, rounding being monotone;
 //   N + P - M + root with M <= N, P is not below max(N, P) but for rounding.
 // The arithmetic of the others is the CPU code's, in FP32 (this file is built
@@ -302,9 +303,12 @@ __global__ void pod_seed(PodArgs a, const float *__restrict__ src, int nshot, fl
     const float t0 = dist * a.S[iz + (long long)ix * g.nz + (long long)iy * g.nx * g.nz];
     float *Ts = a.T + (long long)s * 2 * g.vol;
     const long long c = (iz + 1) + (long long)(ix + 1) * g.pz + (long long)(iy + 1) * g.px * g.pz;
-    Ts[c] = -t0;
+    // a source later than unreached times lowers no cell, and is not one of the
+    // cells that step 0 may lower: no front
+    const bool front = t0 < 1e6f;
+    Ts[c] = front ? -t0 : t0;
     Ts[g.vol + c] = t0;
-    if (a.nit[s] <= 0) return;
+    if (!front || a.nit[s] <= 0) return;
     const int seg = s % kSeg;
     for (int dy1 = -1; dy1 <= 1; dy1++)
         for (int dx1 = -1; dx1 <= 1; dx1++)
