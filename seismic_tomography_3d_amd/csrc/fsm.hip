@@ -257,6 +257,7 @@ __global__ __launch_bounds__(256) void fsm_test(const float *__restrict__ T,
     const float *Tk = Ts + plane * (y1 - w.ty), *Sk = S + plane * (y1 - w.ty - by);
     float u00 = Tk[t00], u10 = Tk[t10], u01 = Tk[t01], u11 = Tk[t11];
     float v00 = Sk[s00], v10 = Sk[s10], v01 = Sk[s01], v11 = Sk[s11];
+    float ubig = tmag3(tmag3(u00, u10, u01), u11, u11);
     bool hit = false;
     for (int c = 0; c < nc; c++) {
         const int k = y1 + w.ty * c;
@@ -279,8 +280,11 @@ __global__ __launch_bounds__(256) void fsm_test(const float *__restrict__ T,
         f.se = pmin(f.sve, pmin(m01, v01));
         f.sn = pmin(f.svn, pmin(v01, v00));
         f.s = v11;
-        const float res = FAST ? fsm_update_fast<true>(n00, f, on, g) : fsm_update_any(n00, f, g);
+        const float nbig = tmag3(n10, n01, n11);
+        const float res = FAST ? fsm_update_fast<true>(n00, f, on, g, tmag3(nbig, ubig, ubig))
+                               : fsm_update_any(n00, f, g);
         hit |= !(res == n00);
+        ubig = tmag3(nbig, n00, n00);
         u00 = n00;
         u10 = n10;
         u01 = n01;

@@ -61,13 +61,13 @@ inline FsmGeo fsm_geometry(int nx, int ny, int nz, float dx, float dy, float dz)
 
 // Whether the FAST update's ranges hold: spacings and their squares far from
 // under- and overflow and within a factor of 1000 of each other (the slack of
-// its 2D bound), times of ordinary size, root arguments 0 or of 2^-101 and more:
-// an argument is (s / d)^2 times at least 8 less another number, and where the
-// two cancel, a multiple of 2^-25 of it.
+// its 2D bound); root arguments 0 or of 2^-101 and more (an argument is (s / d)^2
+// times at least 8 less another number, and where the two cancel, a multiple of
+// 2^-25 of it); no time above the 1e6 of unreached cells, not even the seeds'.
 inline bool fsm_fast(const FsmGeo &g, float slow_min, float slow_max) {
     const float lo = std::min({g.dx, g.dy, g.dz}), hi = std::max({g.dx, g.dy, g.dz});
     return lo > 1e-6f && hi < 1e6f && hi < 1000.0f * lo && slow_min > 1e-9f &&
-           slow_min > 1e-11f * hi && slow_max < 1e4f;
+           slow_min > 1e-11f * hi && slow_max < 1e4f && slow_max * hi < 1e5f;
 }
 
 // Upwind travel times of a cell (v along z, e along x, n along y and their
@@ -79,13 +79,50 @@ struct FsmIn {
     float sv, se, sn, sve, svn, sen, s;
 };
 
-// Least of floats that are never negative nor NaN: their bit patterns order as
-// integers, and an integer minimum needs no quieting of its operands.
+// Least of slownesses, which are never negative nor NaN: their bit patterns order
+// as integers, and an integer minimum needs no quieting of its operands.
 __device__ __forceinline__ float pmin(float a, float b) {
     return __int_as_float(min(__float_as_int(a), __float_as_int(b)));
 }
-__device__ __forceinline__ float pmax(float a, float b) {
-    return __int_as_float(max(__float_as_int(a), __float_as_int(b)));
+// The same of times, which can be negative (beside a source the 3D operator gives
+// such times where spacings and slownesses differ much).  A NaN is left out.  The
+// instructions by name: the compiler would first quiet every time that was loaded.
+__device__ __forceinline__ float tmin(float a, float b) {
+#if defined(__AMDGCN__)
+    float r;
+    asm("v_min_f32 %0, %1, %2" : "=v"(r) : "v"(a), "v"(b));
+    return r;
+#else
+    return __builtin_fminf(a, b);
+#endif
+}
+__device__ __forceinline__ float tmin3(float a, float b, float c) {
+#if defined(__AMDGCN__)
+    float r;
+    asm("v_min3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return __builtin_fminf(a, __builtin_fminf(b, c));
+#endif
+}
+__device__ __forceinline__ float tmax3(float a, float b, float c) {
+#if defined(__AMDGCN__)
+    float r;
+    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return __builtin_fmaxf(a, __builtin_fmaxf(b, c));
+#endif
+}
+// the largest magnitude
+__device__ __forceinline__ float tmag3(float a, float b, float c) {
+#if defined(__AMDGCN__)
+    float r;
+    asm("v_max3_f32 %0, |%1|, |%2|, |%3|" : "=v"(r) : "v"(a), "v"(b), "v"(c));
+    return r;
+#else
+    return tmax3(__builtin_fabsf(a), __builtin_fabsf(b), __builtin_fabsf(c));
+#endif
 }
 
 // The arms of the 3D operator.  Products with 0.5 are exact, so the fused
@@ -172,14 +209,15 @@ __device__ float fsm_update_any(float T, const FsmIn &c, const FsmGeo &g) {
 // masked by selects.  A walk's lanes are cells that change, where some lane
 // needs each operator at nearly every step: without the tests a lone shot's
 // launch takes 16 us instead of 19, 64 shots 25.5 ms instead of 27.5.
+// big, with PRUNE: at least the largest magnitude of the upwind times.
 template <bool PRUNE>
 __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool on,
-                                                 const FsmGeo &g) {
+                                                 const FsmGeo &g, float big = 0.0f) {
     const float dx = g.dx, dy = g.dy, dz = g.dz;
     const float tv = c.tv, te = c.te, tn = c.tn;
-    const float t1D = pmin(tv + dz * c.sv, pmin(te + dx * c.se, tn + dy * c.sn));
-    const float latest = pmax(tv, pmax(te, tn));
-    const float lim = pmin(T, t1D);
+    const float t1D = tmin3(tv + dz * c.sv, te + dx * c.se, tn + dy * c.sn);
+    const float latest = tmax3(tv, te, tn);
+    const float lim = tmin(T, t1D);
     bool try3 = true, pxz = true, pyz = true, pxy = true;
     if (PRUNE) {
         float l3 = __builtin_fmaf(g.wv, tv, c.tnve);
@@ -188,8 +226,7 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
         l3 = __builtin_fmaf(g.wev, c.tev, l3);
         l3 = __builtin_fmaf(g.wen, c.ten, l3);
         l3 = __builtin_fmaf(g.wnv, c.tnv, l3);
-        const float big = pmax(pmax(latest, c.tnve), pmax(c.tev, pmax(c.ten, c.tnv)));
-        const float far = __builtin_fmaf(big + lim, 7.6293945e-6f, lim);
+        const float far = __builtin_fmaf(big + __builtin_fabsf(lim), 7.6293945e-6f, lim);
         try3 = on & (t1D > latest) & (l3 < far);
         pxz = try3 | (on & (__builtin_fmaf(c.sve, g.dmin, c.tev) < far));
         pyz = try3 | (on & (__builtin_fmaf(c.svn, g.dmin, c.tnv) < far));
@@ -220,8 +257,10 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
         const float t = div_rn((ta * g.dx2i + tb * g.dy2i) + sqrt_rn(q), g.xy, g.rxy);
         xy = ok ? t : xy;
     }
-    const float t2D = smin(xz, smin(yz, xy));
-    const bool use3 = try3 & (smin(t1D, t2D) > latest);
+    // (with PRUNE a NaN of the xz plane, with which the cell is not lowered, is
+    // left out)
+    const float t2D = PRUNE ? tmin(xz, smin(yz, xy)) : smin(xz, smin(yz, xy));
+    const bool use3 = try3 & (t1D > latest) & !(t2D <= latest);
     if (!PRUNE || __any(use3)) {
         float ta, tb, tc;
         fsm_arms(c, ta, tb, tc);
@@ -230,9 +269,9 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
                          g.dx2dy2 * (ta - tc) * (ta - tc);
         const float t1 = tb * g.dz2i + ta * g.dx2i + tc * g.dy2i;
         const float t = div_rn(t1 + sqrt_rn(t2 - t3), g.dsum, g.rdsum);
-        t3D = use3 & (t2 >= t3) ? t : t3D;
+        t3D = (use3 & (t2 >= t3)) ? t : t3D;
     }
-    return smin(lim, smin(t2D, t3D));
+    return PRUNE ? tmin3(lim, t2D, t3D) : smin(lim, smin(t2D, t3D));
 }
 
 }  // namespace st

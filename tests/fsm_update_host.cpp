@@ -7,13 +7,13 @@
 // (with 0 draws: a list of ordinary ones).  For each set of units,
 // neighbourhoods of the kinds the sweeps meet: partly unreached ones (1e6),
 // passing fronts at a distance of up to 10^5 cells, times at the edges of the
-// operators' ranges to the last bit, and arbitrary ones.  walk: the form of the
-// blocks' walk must equal the general one in every bit; test: the form with
-// operators left out must lower every cell the general one lowers; roots: as
-// walk, with units of the least slowness to spacing and one time of each
-// neighbourhood moved to where the argument of the 3D operator's root is a few
-// units of its last place.  Prints what differs and the counts; fails if any
-// does.
+// operators' ranges to the last bit, and arbitrary ones, negative among them.
+// walk: the form of the blocks' walk must equal the general one in every bit;
+// test: the form with operators left out must lower every cell the general one
+// lowers; roots: as walk, with units of the least slowness to spacing and one
+// time of each neighbourhood moved to where the argument of the 3D operator's
+// root is a few units of its last place.  Prints what differs and the counts;
+// fails if any does.
 #include <cmath>
 #include <cstdio>
 #include <cstdlib>
@@ -92,9 +92,12 @@ FsmIn neighbourhood(const Units &u, float &T) {
         c.tn = pick(2) ? ulps(c.tv + u.dz * c.svn, pick(9) - 4)
                        : ulps(c.te + u.dx * c.sen, pick(9) - 4);
         break;
-    case 2:   // rough times
-        for (float *p : t) *p = (float)std::max(0.0, *p + uni(-1, 1) * step * logu(1e-4, 10));
+    case 2: {   // rough times, some negative
+        const double least = pick(2) ? 0.0 : -1e30, by = logu(1e-4, 10);
+        for (float *p : t) *p = (float)std::max(least, *p + uni(-1, 1) * step * by);
+        if (pick(2)) T = (float)std::max(least, T + uni(-1, 1) * step * by);
         break;
+    }
     case 3:   // as they come, a few units off
         for (float *p : t) *p = ulps(*p, pick(7) - 3);
         break;
@@ -102,12 +105,19 @@ FsmIn neighbourhood(const Units &u, float &T) {
     }
     switch (pick(4)) {   // the cell's own time: unreached, or near the arrival
     case 0: T = 1e6f; break;
-    case 1: T = std::max(0.0f, fsm_update_any(1e6f, c, fsm_geometry(2, 2, 2, u.dx, u.dy, u.dz)));
+    case 1: T = fsm_update_any(1e6f, c, fsm_geometry(2, 2, 2, u.dx, u.dy, u.dz));
             T = ulps(T, pick(7) - 3); break;
-    case 2: T = (float)std::max(0.0, T + uni(-1, 1) * step * logu(1e-5, 10)); break;
+    case 2: T = (float)(T + uni(-1, 1) * step * logu(1e-5, 10)); break;
     default: break;
     }
+    for (float *p : t) *p = std::min(*p, 1e6f);   // no time is above unreached ones
+    T = std::min(T, 1e6f);
     return c;
+}
+
+float test_update(float T, const FsmIn &c, const FsmGeo &g) {
+    const float big = tmag3(tmag3(c.tv, c.te, c.tn), tmag3(c.tev, c.ten, c.tnv), c.tnve);
+    return fsm_update_fast<true>(T, c, true, g, big);
 }
 
 // t2 - t3 of the 3D operator, as the update has them
@@ -168,7 +178,7 @@ int main(int argc, char **argv) {
             FsmIn c = neighbourhood(u, T);
             if (roots) cancel_root(c, g);
             const float a = fsm_update_any(T, c, g), b = walk ? fsm_update_fast<false>(T, c, true, g)
-                                                             : fsm_update_fast<true>(T, c, true, g);
+                                                             : test_update(T, c, g);
             all++;
             if (walk ? std::memcmp(&a, &b, 4) == 0 : a == T || b != T) continue;
             if (bad++ < 20)
