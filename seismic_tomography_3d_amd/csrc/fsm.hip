@@ -40,10 +40,11 @@
 // the launch itself) and there are (blocks along the longest diagonal) of
 // them per sweep; a batch adds the vector issue of the busiest SIMD.
 // Measured: one shot of 121 x 97 x 61 cells 21.1 ms with a launch per plane of
-// cells, 6.5 with all blocks walked, 5.0 now; 64 shots of 201 x 201 x 101 77.5,
-// 39.2, 25.5 ms (walks 20, tests 5.6).  Blocks of 9 / 11 / 14 / 15 / 22 cells of
-// z: 26.7 / 25.9 / 25.5 / 25.5 / 26.9 ms for the 64 shots, 4.8 / 4.9 / 5.0 /
-// 5.0 / 5.4 for the lone one.
+// cells, 6.5 with all blocks walked, 4.4 to 5.2 now (by the model); 64 shots of
+// 201 x 201 x 101 77.5, 39.2, 25.9 ms (walks 19.5, tests 5.7).  Blocks of 9 / 11 /
+// 14 / 15 / 22 cells of z, before the update followed negative roots and times
+// (25.5 ms): 26.7 / 25.9 / 25.5 / 25.5 / 26.9 ms for the 64 shots, 4.8 / 4.9 / 5.0
+// / 5.0 / 5.4 for the lone one.
 //
 // Layout: one padded volume per shot, z fastest.
 //

@@ -615,7 +615,7 @@ __global__ __launch_bounds__(256) void conv3d_bwd_w(const float *__restrict__ X,
     }
 #pragma unroll
     for (int i = 0; i < TW; i++) {
-        const int tap = KS == 1 ? 0 : w + 4 * i;
+        const int tap = w + 4 * i;
         if (tap >= TAPS) break;
 #pragma unroll
         for (int j = 0; j < CT; j++)

@@ -727,8 +727,9 @@ void wave_shots(st_ctx *ctx, const float *wavelet, int nt, const float *src_xyz,
     a.ntz = (w.nzz - 4 + TZ - 1) / TZ;
     a.ntx = (nxi + TXT - 1) / TXT;
     const long long tiles = (long long)a.ntz * a.ntx;
-    // shots per launch: enough workgroups (about 2048, 8 per CU) with chunks
-    // of at least 32 planes; two wavefields per shot, at most 24 GiB
+    // shots per launch: as many as it takes for about 2048 workgroups (8 per CU)
+    // with chunks of 32 planes, whatever chunk length is then chosen below; two
+    // wavefields per shot, at most 24 GiB
     int G = group;
     if (G == 0) {
         const long long wg1 = tiles * std::max(1, nyi / 32);
@@ -737,7 +738,8 @@ void wave_shots(st_ctx *ctx, const float *wavelet, int nt, const float *src_xyz,
     G = std::min(G, nshot);
     G = (int)std::max<long long>(1, std::min<long long>(G, (24LL << 30) / (8 * N)));
     // planes per workgroup: the chunk length that is done first.  Three
-    // workgroups fit a CU, so they run in rounds of 3 ncu; a last round with
+    // workgroups fit a CU (157 registers for either tile width; the weights below
+    // are measured for three), so they run in rounds of 3 ncu; a last round with
     // two or one left per CU takes 0.73 or 0.5 of a full one's time.  A chunk
     // of y planes costs y + 2 plane times (the ring's first planes are read
     // before the first step).  Measured, us per step at y planes:
