@@ -189,7 +189,8 @@ __device__ float fsm_update_any(float T, const FsmIn &c, const FsmGeo &g) {
 // the source across spacings that differ much.  The code's result is then a
 // NaN, and std::min keeps its first argument if either is one: the operators
 // are combined here in the code's order with the code's operands, so that a NaN
-// takes the same others with it.
+// takes the same others with it.  The 3D operator comes last: with a NaN before it
+// it is dropped, and the 1e6 it stands at where it does not apply offers nothing.
 //
 // PRUNE, with lim the least of the cell's time and the 1D operators:
 // * t3D is at least the weighted mean of its arms (its root is not negative
@@ -232,7 +233,7 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
         pyz = try3 | (on & (__builtin_fmaf(c.svn, g.dmin, c.tnv) < far));
         pxy = try3 | (on & (__builtin_fmaf(c.sen, g.dmin, c.ten) < far));
     }
-    float xz = 1e6f, yz = 1e6f, xy = 1e6f, t3D = 1e6f;
+    float xz = 1e6f, yz = 1e6f, xy = 1e6f;
     if (!PRUNE || __any(pxz)) {
         const bool ok = pxz & (tv < te + dx * c.sve) & (te < tv + dz * c.sve);
         const float ta = c.tev + te - tv;
@@ -260,7 +261,8 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
     // (with PRUNE a NaN of the xz plane, with which the cell is not lowered, is
     // left out)
     const float t2D = PRUNE ? tmin(xz, smin(yz, xy)) : smin(xz, smin(yz, xy));
-    const bool use3 = try3 & (t1D > latest) & !(t2D <= latest);
+    const bool use3 = try3 & (t1D > latest) & (t2D > latest);   // not with a NaN
+    const float res = PRUNE ? tmin(lim, t2D) : smin(lim, t2D);
     if (!PRUNE || __any(use3)) {
         float ta, tb, tc;
         fsm_arms(c, ta, tb, tc);
@@ -269,9 +271,9 @@ __device__ __forceinline__ float fsm_update_fast(float T, const FsmIn &c, bool o
                          g.dx2dy2 * (ta - tc) * (ta - tc);
         const float t1 = tb * g.dz2i + ta * g.dx2i + tc * g.dy2i;
         const float t = div_rn(t1 + sqrt_rn(t2 - t3), g.dsum, g.rdsum);
-        t3D = (use3 & (t2 >= t3)) ? t : t3D;
+        return (use3 & (t2 >= t3) & (t < res)) ? t : res;
     }
-    return PRUNE ? tmin3(lim, t2D, t3D) : smin(lim, smin(t2D, t3D));
+    return res;
 }
 
 }  // namespace st
